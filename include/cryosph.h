@@ -185,8 +185,10 @@ int cryo_ensemble_run_steps(cryo_solver* const* solvers, int32_t count, int64_t 
 
 /* Extension (no counterpart in the reference, whose CUDA kernels have one launch
  * shape): the launch variant of the interface and forces passes, bit 0 set =
- * forces by per-particle neighbour-list gathers instead of LDS-staged cell
- * tiles, bit 1 set = the same for the interface pass.  Every variant gives the
+ * the forces pass with the other number of lanes per particle (two where its
+ * size rule takes four, four where it takes two), bit 1 set = the interface
+ * pass by per-particle neighbour-list gathers instead of LDS-staged cell tiles
+ * (SPS and Akinci runs; others have one form).  Every variant gives the
  * same results bit for bit; only the speed differs with tank size and fill.
  * cryo_solver_autotune times `trial_steps` steps of each variant from the
  * solver's current state (after one untimed step each), keeps the fastest,
@@ -225,7 +227,7 @@ int cryo_solver_launch_variant(cryo_solver* s, int32_t* variant);
 int cryo_solver_autotune(cryo_solver* s, int32_t trial_steps, int32_t* variant, double* ms_per_step);
 
 /* Extension (no counterpart in the reference): the cell-tile shape of the
- * LDS-staged interface and forces passes, in grid cells along x, y and z
+ * LDS-staged interface pass (SPS and Akinci runs), in grid cells along x, y and z
  * (default 3 x 3 x 3).  Accepted: 1 <= x <= 16, y, z >= 1, (y + 2)(z + 2) <= 25
  * and y z <= 9; other shapes fail with CRYO_ERR_INVALID_ARGUMENT.  Every shape
  * gives the same results bit for bit; the shape sets how many particles each

@@ -26,7 +26,8 @@ CSRC = HERE / "csrc"
 OBJ = HERE / "_build"
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
-LIB_SOURCES = ["kernels_grid.hip", "kernels_physics.hip", "kernels_step.hip", "kernels_adjoint.hip", "solver.cpp",
+LIB_SOURCES = ["kernels_forces_akinci.hip", "kernels_forces_csf.hip", "kernels_forces_none.hip", "kernels_grid.hip",
+               "kernels_physics.hip", "kernels_step.hip", "kernels_adjoint.hip", "solver.cpp",
                "geometry.cpp", "io.cpp"]
 COMMON = ["-O3", "-fPIC", "-std=c++17", "-ffp-contract=off", "-Wno-unknown-pragmas",
           f"-I{ROOT / 'include'}", f"-I{CSRC}"]

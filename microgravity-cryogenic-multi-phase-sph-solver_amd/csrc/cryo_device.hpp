@@ -164,6 +164,38 @@ __host__ __device__ inline float akinci_coh(float r, float c) {
   return coeff * (2.0f * base - c3 * c3 / 64.0f);
 }
 
+// ------------------------------- correctly rounded division and square root
+// The IEEE sequences the compiler emits for x / y and sqrtf carry range
+// scaling and special cases: 43 and 54 issue cycles per wave here, where a
+// plain multiply or FMA takes 3 (measured, 2 or more waves per SIMD).  In the
+// range the pair loops work in the same correctly rounded results follow from
+// FMA residuals (P. Markstein, "Computation of elementary functions on the IBM
+// RISC System/6000 processor", IBM J. Res. Dev. 34, 1990): 30 cycles for the
+// square root, 14 for a reciprocal that several quotients share, 15 a quotient.
+// y: normal, at most 2^126; x: 0 or at least kFastLow in magnitude, the quotient normal.
+struct Recip {
+  float y, r;  // r: 1 / y correctly rounded
+};
+__device__ inline Recip recip_rn(float y) {
+  const float r0 = __builtin_amdgcn_rcpf(y);
+  return Recip{y, __builtin_fmaf(__builtin_fmaf(-y, r0, 1.0f), r0, r0)};
+}
+__device__ inline float div_rn(float x, const Recip& R) {
+  const float q0 = x * R.r;
+  const float q1 = __builtin_fmaf(__builtin_fmaf(-R.y, q0, x), R.r, q0);  // within one ulp
+  return __builtin_fmaf(__builtin_fmaf(-R.y, q1, x), R.r, q1);
+}
+// x: normal, within [2^-96, 2^126]
+__device__ inline float sqrt_rn(float x) {
+  const float y = __builtin_amdgcn_rsqf(x);
+  float g = x * y, h = 0.5f * y;
+  const float e = __builtin_fmaf(-h, g, 0.5f);
+  g = __builtin_fmaf(g, e, g);
+  h = __builtin_fmaf(h, e, h);
+  return __builtin_fmaf(__builtin_fmaf(-g, g, x), h, g);
+}
+constexpr uint32_t kFastLow = 0x0d800000u;  // 2^-100, smallest numerator of div_rn
+
 // Element k (0 or 1) of a two-entry table without indexing it: a dynamic
 // index into a by-value parameter struct would put the struct in scratch.
 template <class T>
@@ -184,6 +216,9 @@ struct SimParams {
   // harmonic viscosity 2 mu_a mu_b / (mu_a + mu_b) of the phase pairs LL, LV,
   // VV (0 when mu_a + mu_b = 0), evaluated once in the pair loops' order
   float eta_ll, eta_lv, eta_vv;
+  // pair conductivity 4 k_i k_j / (k_i + k_j) of a target and a neighbour of
+  // given phases, the same way
+  float k_ll, k_lv, k_vl, k_vv;
   int density_mode, no_slip, sps, tvf, tvf_stress;
   float tvf_factor, tvf_sigma_min, shift_strength;
   int tvf_interface_only;
@@ -197,6 +232,10 @@ struct SimParams {
       split_ratio, heat_power;
   int has_vapor;
   int compensated;  // compensated neighbour sums (precision form)
+  // the pair loops' fast division and square root: allowed for this smoothing
+  // length (fast), for pairs with r2 at least r2_fast
+  int fast;
+  float r2_fast;
 };
 
 // ------------------------------------------------------- device state block
@@ -639,6 +678,9 @@ __host__ __device__ inline float df_diff(float a, float al, float b, float bl) {
   const float s = a - b;
   return s + (diff_err(a, b, s) + (al - bl));
 }
+__host__ __device__ inline V3 df_diff3(V3 a, V3 al, V3 b, V3 bl) {
+  return V3{df_diff(a.x, al.x, b.x, bl.x), df_diff(a.y, al.y, b.y, bl.y), df_diff(a.z, al.z, b.z, bl.z)};
+}
 // Pair vector x_i - x_j.  HP = false: the float difference of the stored
 // positions, the reference's arithmetic.  HP = true (the precision form):
 // the double-float positions' difference, to which particle j's low part is
@@ -669,6 +711,16 @@ __host__ __device__ inline void df_add(float& x, float& lo, float d) {
   lo = t - (hi - s);
   x = hi;
 }
+// Everything the forces pass reads of one neighbour, in one 64-byte line, so
+// that a gathered neighbour costs one line of L1 and not one per array.
+// Written once per rates evaluation: fluid by the density pass, walls by the
+// wall pass.
+struct alignas(64) PairRec {
+  float4 x;  // position, phase (int bits)
+  float4 q;  // {p, m, rho, T} fluid; {p, p_wv, rho_tvf, T} wall (as nrec)
+  float4 v;  // velocity, V = m / rho (fluid); no-slip ghost velocity, 0 (wall)
+  float4 t;  // transport velocity, transport volume 1 / sigma (fluid, transport velocity on)
+};
 struct Scratch {
   float4 *a, *ab, *ns, *vw, *fw, *mw;
   float *p, *drho, *dTdt, *sigma, *kappa, *nu_t, *alpha, *wall_w, *heat_w, *out_m, *out_h, *w_norm, *p_wv, *rmin;
@@ -681,6 +733,7 @@ struct Scratch {
   // V = m / rho of each fluid particle for one rates evaluation (density
   // pass): the pair loops read it instead of dividing per pair.
   float* vol;
+  PairRec* rec;
 };
 struct PV {  // kernel view
   Persist s;

@@ -65,7 +65,13 @@ void launch_smooth_normals(const PV& pv, const GridDev& g, const SimParams& P, c
                            hipStream_t s);
 void launch_heat_norm(DevState* st, const double* partials, int nb, bool active, hipStream_t s);
 void launch_forces(const PV& pv, const GridDev& g, const SimParams& P, const NbrList& L, DevState* st, Count n,
-                   bool csf_mode, bool akinci, bool continuity, bool thermal, bool tiled, hipStream_t s);
+                   bool csf_mode, bool akinci, bool continuity, bool thermal, bool other_lanes, hipStream_t s);
+void launch_forces_none(const PV& pv, const GridDev& g, const SimParams& P, const NbrList& L, DevState* st, Count n,
+                        bool continuity, bool thermal, int lanes, hipStream_t s);
+void launch_forces_csf(const PV& pv, const GridDev& g, const SimParams& P, const NbrList& L, DevState* st, Count n,
+                       bool continuity, bool thermal, int lanes, hipStream_t s);
+void launch_forces_akinci(const PV& pv, const GridDev& g, const SimParams& P, const NbrList& L, DevState* st, Count n,
+                          bool continuity, bool thermal, int lanes, hipStream_t s);
 void launch_probe(const PV& pv, const GridDev& g, const SimParams& P, const float* pts, float* out, int np,
                   hipStream_t s);
 void launch_shifting(const PV& pv, const GridDev& g, const SimParams& P, const NbrList& L, const DevState* st, Count n,

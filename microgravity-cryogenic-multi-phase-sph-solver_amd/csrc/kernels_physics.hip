@@ -7,22 +7,17 @@
 //   k_wall_bc    Adami wall extrapolation          (navier_stokes.cu:16-69)
 //   k_interface  colour gradient, alpha, wall/heat weights, contact angle, SPS,
 //                pointwise CSF normals             (surface_tension.cu:5-118, navier_stokes.cu:71-119)
-//   k_forces     transport velocity, momentum with wall loads, CSF or Akinci,
-//                continuity, conduction, dt maxima (SPH_kernels.cu:56-104,162-203,
-//                navier_stokes.cu:121-245, surface_tension.cu:120-213,
-//                phase_change.cu:31-75, sph_solver.cu:62-99)
+//   k_forces     everything else of the rates (kernels_forces.hpp)
 // Every accumulator adds its neighbours in the reference order (ascending
 // sorted index), with the reference's per-pair expressions, so each field is
 // the same float the reference computes (given equal inputs).
-#include "kernels.hpp"
+#include <stdexcept>
+
+#include "pair_lanes.hpp"
 
 namespace cryo {
 
 namespace {
-
-constexpr int kBlock = 256;
-__device__ inline int gtid() { return static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x); }
-inline int blocks_for(long long n) { return static_cast<int>((n + kBlock - 1) / kBlock); }
 
 // Deterministic FP64 block sum: fixed shuffle tree per wave, waves in order.
 __device__ inline void block_sum_store(double v, double* out) {
@@ -37,21 +32,6 @@ __device__ inline void block_sum_store(double v, double* out) {
     *out = s;
   }
 }
-
-// Max of non-negative floats (NaN ignored, as `v > acc ? v : acc` does).
-__device__ inline float wave_max(float v) {
-  for (int off = 32; off > 0; off >>= 1) {
-    const float o = __shfl_down(v, off, 64);
-    v = o > v ? o : v;
-  }
-  return v;
-}
-__device__ inline void atomic_max_nonneg(unsigned* addr, float v) {
-  if (v > 0.0f) atomicMax(addr, __float_as_uint(v));
-}
-
-// pow for positive float arguments: evaluated in double and rounded once.
-__device__ inline float powf_cr(float x, float y) { return static_cast<float>(pow(static_cast<double>(x), static_cast<double>(y))); }
 
 // ------------------------------------------------------- density + EOS
 // Also builds the step's neighbour lists from the same (cell-culled) sweep.
@@ -76,6 +56,13 @@ __global__ __launch_bounds__(kBlock) void k_density(PV pv, GridDev g, SimParams 
       });
     }
     L.count[i] = lw.finish();
+    if (ph != kWall) {  // dead, not yet dropped: what the last evaluation gave it, at its present phase and velocity
+      const float4 v = pv.s.v[i];
+      PairRec& r = pv.t.rec[i];
+      r.x = make_float4(xi.x, xi.y, xi.z, __int_as_float(ph));
+      r.v = make_float4(v.x, v.y, v.z, r.v.w);
+      r.t = st3(ld3(pv.s.vt[i]));
+    }
     return;
   }
   Acc<KS> sum;
@@ -115,8 +102,13 @@ __global__ __launch_bounds__(kBlock) void k_density(PV pv, GridDev g, SimParams 
     p = eos_pressure(P, ph, rho, Ti);
   }
   pv.t.p[i] = p;
-  pv.t.nrec[i] = make_float4(p, mi, rho, Ti);
-  pv.t.vol[i] = mi / rho;
+  const float4 q = make_float4(p, mi, rho, Ti);
+  const float V = mi / rho;
+  pv.t.nrec[i] = q;
+  pv.t.vol[i] = V;
+  const float4 v = pv.s.v[i], vt = pv.s.vt[i];
+  pv.t.rec[i] = PairRec{make_float4(xi.x, xi.y, xi.z, __int_as_float(ph)), q, make_float4(v.x, v.y, v.z, V),
+                        make_float4(vt.x, vt.y, vt.z, P.tvf ? 1.0f / float(sum) : 0.0f)};
 }
 
 // SPH_kernels.cu:36-54 (start-up only).
@@ -209,7 +201,11 @@ __global__ __launch_bounds__(kBlock) void k_wall_bc(PV pv, GridDev g, SimParams 
     const float ratio = (pw[0] - P.p_bg) / P.tait_B + 1.0f;
     rho_tvf = P.rho0[0] * powf_cr(ratio > 0.5f ? ratio : 0.5f, 1.0f / P.tait_gamma);
   }
-  pv.t.nrec[i] = make_float4(pw[0], pw[1], rho_tvf, pv.s.T[i]);
+  const float4 q = make_float4(pw[0], pw[1], rho_tvf, pv.s.T[i]);
+  pv.t.nrec[i] = q;
+  float4 ghost = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  if (P.no_slip && swt > 0.0f) ghost = st3(V3(sv) * (-1.0f / swt));
+  pv.t.rec[i] = PairRec{make_float4(xi.x, xi.y, xi.z, __int_as_float(kWall)), q, ghost, st3(V3{0, 0, 0})};
   pv.t.a[i] = st3(V3{0, 0, 0});
 }
 
@@ -452,351 +448,7 @@ __global__ __launch_bounds__(kBlock) void k_smooth_normals(PV pv, GridDev g, Sim
   pv.t.ns[i] = st3(normalized(V3(acc)));
 }
 
-// ------------------------------------------------------------------ forces
-// What one neighbour contributes to the forces pass.  For a wall neighbour
-// `v` holds its no-slip ghost velocity vw, for a fluid one its velocity; `vt`
-// is the fluid transport velocity (read only when the pass needs it).
-struct NbrData {
-  float4 x;
-  int ph;
-  float4 rec;  // {p, m, rho, T} fluid; {p, p_wv, rho_tvf, T} wall
-  float4 v;
-  float4 vt;
-  float V;   // m / rho (fluid)
-  float Vt;  // 1 / sigma (fluid, transport velocity on)
-};
-
-__device__ inline bool forces_need_vt(const SimParams& P, bool continuity) {
-  return (P.tvf && P.tvf_stress) || (continuity && P.tvf);
-}
-
-// Neighbour data straight from the particle arrays.
-__device__ inline NbrData load_nbr(const PV& pv, const SimParams& P, int j, bool need_vt) {
-  NbrData d;
-  d.x = pv.s.x[j];
-  d.ph = pv.s.phase[j];
-  d.rec = pv.t.nrec[j];
-  d.V = pv.t.vol[j];
-  const float4 v = pv.s.v[j];
-  float4 vw = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  if (P.no_slip) vw = pv.t.vw[j];
-  d.vt = v;
-  if (need_vt) d.vt = pv.s.vt[j];
-  float sig = 1.0f;
-  if (P.tvf) sig = pv.t.sigma[j];
-  // every gather of the pair in flight together, then one wait
-  settle(d.x.x, d.x.y, d.x.z, d.ph, d.rec.x, d.rec.y, d.rec.z, d.rec.w, v.x, v.y, v.z, d.V);
-  if (P.no_slip) settle(vw.x, vw.y, vw.z);
-  if (need_vt) settle(d.vt.x, d.vt.y, d.vt.z);
-  if (P.tvf) settle(sig);
-  d.v = d.ph == kWall ? vw : v;
-  d.Vt = P.tvf && is_fluid(d.ph) ? 1.0f / sig : 0.0f;
-  return d;
-}
-
-// Momentum, wall loads, transport velocity, CSF / Akinci, continuity and
-// conduction rates of particle i, and its dt maxima.  `visit(f)` calls
-// f(j, NbrData) for every neighbour in the reference order.
-// ST: 0 no tension pass, 1 CSF with vapour present, 2 Akinci.
-struct Maxima {
-  float v = 0.0f, a = 0.0f, tv = 0.0f, nu = 0.0f, sp = 0.0f;
-};
-template <int ST, bool CONT, bool THERMAL, bool KS, class Visit>
-__device__ inline void forces_particle(const PV& pv, const SimParams& P, DevState* st, int i, Visit&& visit,
-                                       Maxima& mx) {
-  struct {
-    bool csf_mode, akinci, continuity, thermal;
-  } constexpr F{ST == 1, ST == 2, CONT, THERMAL};
-  {
-    const uint8_t ph = pv.s.phase[i];
-    if (!is_fluid(ph)) {
-      pv.t.ab[i] = st3(V3{0, 0, 0});
-      pv.t.a[i] = st3(V3{0, 0, 0});
-      pv.t.fw[i] = st3(V3{0, 0, 0});
-      pv.t.mw[i] = st3(V3{0, 0, 0});
-      if (F.continuity) pv.t.drho[i] = 0.0f;
-      if (F.thermal) pv.t.dTdt[i] = 0.0f;
-    } else {
-      const V3 grav = st->gravity;
-      const float dt_now = st->dt;
-      const int pi_idx = pidx(ph);
-      const V3 xi = ld3(pv.s.x[i]);
-      const V3 li = pos_lo<KS>(pv.s.xlo, i);
-      const V3 vi = ld3(pv.s.v[i]);
-      const float mi = pv.s.m[i];
-      const float rhoi = pv.s.rho[i];
-      const float Ti = pv.s.T[i];
-      const float sigmai = pv.t.sigma[i];
-      const float Vi = mi / rhoi;
-      const float Vi2 = Vi * Vi;
-      const float pi = pv.t.p[i];
-      const float ci = sound_speed(P, ph, Ti);
-      const float h = P.kernel.h;
-      const float eta2 = 0.01f * h * h;
-      // transport velocity (SPH_kernels.cu:56-104)
-      const bool tvf_on = P.tvf && !(sigmai < P.tvf_sigma_min) &&
-                          !(P.tvf_interface_only && !(pv.t.alpha[i] > 0.0f));
-      const float Vt = 1.0f / sigmai;
-      const float Vt2 = Vt * Vt;
-      const float mt = rhoi * Vt;
-      const float pb = P.tvf_factor * sel2(P.rho0, pi_idx) * ci * ci;
-      const float inv_gamma = 1.0f / P.tait_gamma;
-      AccV3<KS> sum_t;
-      // momentum (navier_stokes.cu:121-245)
-      const float etai = sel2(P.mu, pi_idx) + (P.sps ? rhoi * pv.t.nu_t[i] : 0.0f);
-      const float alpha_i = ph == kVapor ? P.alpha_av_vap : P.alpha_av;
-      AccV3<KS> force, acc_av;
-      const float r_guard = 0.6f * P.dx;
-      const bool tvf_stress = P.tvf && P.tvf_stress;
-      const V3 dvi = ld3(pv.s.vt[i]) - vi;
-      AccV3<KS> fwall, mwall;
-      const V3 origin = st->origin;
-      // CSF (surface_tension.cu:120-177)
-      const V3 ni = F.csf_mode ? ld3(pv.t.ns[i]) : V3{0, 0, 0};
-      const bool csf_on = F.csf_mode && norm2(ni) > 0.25f;
-      const float cci = ph == kLiquid ? 1.0f : 0.0f;
-      Acc<KS> num, den;
-      AccV3<KS> G;
-      // Akinci (surface_tension.cu:179-213)
-      const bool ak_on = F.akinci && ph == kLiquid;
-      const V3 nak = ak_on ? ld3(pv.s.nrm[i]) : V3{0, 0, 0};
-      const float psi = P.rho0[0] * P.vol0;
-      AccV3<KS> acc_ak;
-      // continuity (SPH_kernels.cu:162-203)
-      const float4* vel = P.tvf ? pv.s.vt : pv.s.v;
-      const V3 vci = F.continuity ? ld3(vel[i]) : V3{0, 0, 0};
-      Acc<KS> div, diff;
-      // conduction (phase_change.cu:31-75)
-      const float ki = sel2(P.k, pi_idx);
-      const bool iso = P.wall_bc == 1;
-      Acc<KS> q;
-
-      visit([&](int j, NbrData d) {
-        if (j == i) return;
-        const V3 xj = ld3(d.x);
-        const int phj = d.ph;
-        const float4 rec = d.rec;
-        const V3 rij = pos_diff<KS>(xi, li, xj, pv.s.xlo, j);
-        const float r2 = norm2(rij);
-        if (r2 >= P.support2) return;
-        const float r = sqrtf(r2);
-        const float dW = kdW(P.kernel, r);
-        const bool separated = r > 1e-12f * h;
-        const V3 gw = separated ? rij * (dW / r) : V3{0, 0, 0};
-        const float Tj = rec.w;
-        if (phj == kWall) {
-          const float pj = rec.x, pwv = rec.y;
-          if (tvf_on) {
-            float rho_w;
-            if (ph == kVapor) {
-              rho_w = (pwv - (P.p_bg - P.vapor_K)) / (P.gas_R * Ti);
-            } else {
-              rho_w = rec.z;  // the wall pass stored rho0 * max(ratio, 0.5)^(1/gamma) here
-            }
-            const float Vj = rho_w > 0.0f ? Vt * rhoi / rho_w : Vt;
-            sum_t += gw * (Vt2 + Vj * Vj);
-          }
-          {
-            const float Vj = P.vol0;
-            const float vsum = Vi2 + Vj * Vj;
-            const float pw = ph == kVapor ? pwv : pj;
-            auto wall_terms = [&](auto& fo, auto& ac) {
-              fo -= gw * (vsum * 0.5f * (pi + pw));
-              if (tvf_stress) fo += vi * (0.5f * vsum * rhoi * dot(dvi, gw));
-              if (r < r_guard && separated) {
-                const float qg = 1.0f - r / r_guard;
-                const V3 nn = rij / r;
-                ac += nn * (4.0f * ci * ci * qg * qg / r_guard);
-                const float vn = dot(vi, nn);
-                if (vn < 0.0f && dt_now > 0.0f) ac -= nn * (qg * vn / dt_now);
-              }
-              if (P.no_slip) {
-                const V3 vij = vi - ld3(d.v);
-                if (separated) fo += vij * (vsum * etai * dW / r);
-                const float vr = dot(vij, rij);
-                if (alpha_i > 0.0f && vr < 0.0f) {
-                  const float mu_ij = h * vr / (r2 + eta2);
-                  const float Pi = -alpha_i * ci * mu_ij / rhoi;
-                  ac -= gw * (rhoi * P.vol0 * Pi);
-                }
-              }
-            };
-            V3 dF;
-            if constexpr (KS) {  // the pair's own terms, added once to each sum
-              V3 df{0, 0, 0}, da{0, 0, 0};
-              wall_terms(df, da);
-              force += df;
-              acc_av += da;
-              dF = df + da * mi;
-            } else {  // the reference's wall load: what the pair changed
-              const V3 f_before = force, a_before = acc_av;
-              wall_terms(force, acc_av);
-              dF = (V3(force) - f_before) + (V3(acc_av) - a_before) * mi;
-            }
-            fwall += dF;
-            mwall += cross(xj - origin, dF);
-          }
-          if (ak_on && r2 > 0.0f) {
-            const float arg = -4.0f * r * r / P.kernel.support + 6.0f * r - 2.0f * P.kernel.support;
-            float adh = 0.0f;
-            if (!(r >= P.kernel.support || 2.0f * r <= P.kernel.support) && arg > 0.0f)
-              adh = P.ak_adh_scale * powf_cr(arg, 0.25f);
-            acc_ak -= (rij / r) * (P.ak_beta * psi * adh);
-          }
-          if (F.continuity) div += P.vol0 * dot(vci, gw);
-          if (F.thermal && iso) {
-            const float rgw = r * dW;
-            q += Vi * P.vol0 * (2.0f * ki) * (Ti - Tj) * rgw / (r2 + eta2);
-          }
-          return;
-        }
-        // fluid neighbour
-        const float pj = rec.x, mj = rec.y, rhoj = rec.z;
-        if (tvf_on) {
-          const float Vj = d.Vt;  // 1 / sigma_j
-          sum_t += gw * (Vt2 + Vj * Vj);
-        }
-        const float Vj = d.V;  // mj / rhoj, divided once per particle
-        const float vsum = Vi2 + Vj * Vj;
-        const float pt = (rhoj * pi + rhoi * pj) / (rhoi + rhoj);
-        force -= gw * (vsum * pt);
-        const V3 vj = ld3(d.v);
-        if (tvf_stress) {
-          const V3 Ag = vi * (rhoi * dot(dvi, gw)) + vj * (rhoj * dot(ld3(d.vt) - vj, gw));
-          force += Ag * (0.5f * vsum);
-        }
-        const V3 vij = vi - vj;
-        const float etaj = sel2(P.mu, pidx(phj)) + (P.sps ? rhoj * pv.t.nu_t[j] : 0.0f);
-        const float eta_sum = etai + etaj;
-        if (eta_sum > 0.0f && separated) {
-          const float eta_ij = P.sps ? 2.0f * etai * etaj / eta_sum
-                                     : (ph == phj ? (ph == kLiquid ? P.eta_ll : P.eta_vv) : P.eta_lv);
-          force += vij * (vsum * eta_ij * dW / r);
-        }
-        if (alpha_i > 0.0f && phj == ph) {
-          const float vr = dot(vij, rij);
-          if (vr < 0.0f) {
-            const float cj = sound_speed(P, phj, Tj);
-            const float mu_ij = h * vr / (r2 + eta2);
-            const float Pi = -alpha_i * 0.5f * (ci + cj) * mu_ij / (0.5f * (rhoi + rhoj));
-            acc_av -= gw * (mj * Pi);
-          }
-        }
-        if (csf_on && is_fluid(phj)) {
-          const V3 gwc = rij * (dW / r);
-          const V3 nj = ld3(pv.t.ns[j]);
-          if (norm2(nj) > 0.25f) {
-            num += Vj * dot(ni - nj, gwc);
-            den += Vj * r * (-dW);
-          }
-          if (P.csf_balanced) {
-            const float cj = phj == kLiquid ? 1.0f : 0.0f;
-            G += gwc * ((Vi * Vi + Vj * Vj) * (rhoj * cci + rhoi * cj) / (rhoi + rhoj));
-          }
-        }
-        if (ak_on && r2 > 0.0f && phj == kLiquid) {
-          const V3 rhat = rij / r;
-          const float K = 2.0f * P.rho0[0] / (rhoi + rhoj);
-          const V3 f_coh = rhat * (-P.ak_gamma * mi * mj * akinci_coh(r, P.kernel.support));
-          const V3 f_curv = (nak - ld3(pv.s.nrm[j])) * (-P.ak_gamma * mi);
-          acc_ak += (f_coh + f_curv) * (K / mi);
-        }
-        if (F.continuity) {
-          div += Vj * dot(vci - (P.tvf ? ld3(d.vt) : vj), gw);
-          if (phj == ph) diff += Vj * 2.0f * (rhoj - rhoi) * dot(-rij, gw) / (r2 + eta2);
-        }
-        if (F.thermal) {
-          const float kj = sel2(P.k, pidx(phj));
-          const float kij = 4.0f * ki * kj / (ki + kj);
-          const float rgw = r * dW;
-          q += Vi * Vj * kij * (Ti - Tj) * rgw / (r2 + eta2);
-        }
-      });
-
-      const V3 ab = tvf_on ? V3(sum_t) * (-pb / mt) : V3{0, 0, 0};
-      pv.t.ab[i] = st3(ab);
-      V3 acc = grav + V3(force) / mi + V3(acc_av);
-      if (st->frame_rot) {
-        const V3 om = st->omega, omd = st->omega_dot;
-        const V3 rr = xi - origin;
-        acc -= cross(omd, rr) + cross(om, cross(om, rr)) + cross(om, vi) * 2.0f;
-      }
-      if (F.csf_mode) {
-        if (csf_on) {
-          const float kappa = float(den) > 0.0f ? 3.0f * float(num) / float(den) : 0.0f;
-          pv.t.kappa[i] = kappa;
-          if (P.wetting != 0) acc += ld3(pv.t.vw[i]);
-          if (P.csf_balanced) {
-            acc += V3(G) * (P.sigma * kappa / mi);
-          } else {
-            const float coeff = 2.0f * P.sigma / (P.rho0[0] + P.rho0[1]);
-            acc += ld3(pv.s.nrm[i]) * (coeff * kappa);
-          }
-        } else {
-          pv.t.kappa[i] = 0.0f;
-        }
-      }
-      if (ak_on) acc += V3(acc_ak);
-      pv.t.a[i] = st3(acc);
-      pv.t.fw[i] = st3(V3(fwall));
-      pv.t.mw[i] = st3(V3(mwall));
-      if (F.continuity) pv.t.drho[i] = rhoi * float(div) + P.delta_sph * h * P.c0 * float(diff);
-      if (F.thermal) {
-        const float qt = float(q) + P.heat_power * pv.t.heat_w[i] * st->heat_inv_norm;
-        pv.t.dTdt[i] = qt / (mi * sel2(P.cp, pi_idx));
-      }
-      // evaluate_rates maxima (sph_solver.cu:62-99)
-      mx.v = norm(vi);
-      const float na = norm(acc), nb = norm(ab);
-      mx.a = na > nb ? na : nb;
-      if (ph == kVapor) mx.tv = Ti;
-      if (P.sps) mx.nu = pv.t.nu_t[i];
-      const float rm = pv.t.rmin[i] > 0.05f * P.dx ? pv.t.rmin[i] : 0.05f * P.dx;
-      mx.sp = 0.5f * P.dx / rm;
-    }
-  }
-}
-
-__device__ inline void publish_maxima(DevState* st, Maxima mx) {
-  mx.v = wave_max(mx.v);
-  mx.a = wave_max(mx.a);
-  mx.tv = wave_max(mx.tv);
-  mx.nu = wave_max(mx.nu);
-  mx.sp = wave_max(mx.sp);
-  if ((threadIdx.x & 63) == 0) {
-    atomic_max_nonneg(&st->max_bits[0], mx.v);
-    atomic_max_nonneg(&st->max_bits[1], mx.a);
-    atomic_max_nonneg(&st->max_bits[2], mx.tv);
-    atomic_max_nonneg(&st->max_bits[3], mx.nu);
-    atomic_max_nonneg(&st->max_bits[4], mx.sp);
-  }
-}
-
-// SWEEP = false: particles whose neighbour list is complete (count >= 0),
-// neighbour data gathered from the particle arrays.  SWEEP = true: the
-// overflowed ones (count < 0) by the cell sweep, which visits the same
-// neighbours in the same order.  Two instances keep the sweep's code and
-// registers out of the list loop.
-template <int ST, bool CONT, bool THERMAL, bool KS, bool SWEEP>
-__global__ __launch_bounds__(kBlock) void k_forces(PV pv, GridDev g, SimParams P, NbrList L, DevState* st, Count nc) {
-  const int n = nc.get();
-  const int i = gtid();
-  Maxima mx;
-  const int cnt = i < n ? L.count[i] : 0;
-  if (i < n && (cnt < 0) == SWEEP) {
-    const bool need_vt = forces_need_vt(P, CONT);
-    const V3 xi = ld3(pv.s.x[i]);
-    auto gathered = [&](auto&& f) {
-      auto one = [&](int j) { f(j, load_nbr(pv, P, j, need_vt)); };
-      if (SWEEP) for_each_nbr(g, xi, one);
-      else for_each_listed(L, i, cnt, one);
-    };
-    forces_particle<ST, CONT, THERMAL, KS>(pv, P, st, i, gathered, mx);
-  }
-  publish_maxima(st, mx);
-}
-
-// ------------------------------------------------ forces, LDS-staged tiles
+// ------------------------------------------------------ LDS-staged cell tiles
 // One workgroup per tile of 3 x 3 x 3 cells.  Every neighbour of the tile's
 // particles lies in the 5 x 5 x 5 cells around it: up to 25 (z, y) rows, each
 // one contiguous index range of the cell-sorted arrays.  The workgroup copies
@@ -824,19 +476,6 @@ struct TileRows {
   int ntrows;
 };
 
-// Block b of an nblocks grid -> the tile it runs.  The hardware deals
-// workgroups round-robin to the 8 XCDs (XCD b % 8); within each group of
-// 8 x kTileChunk blocks, XCD x runs the chunk of kTileChunk consecutive tiles
-// [x kTileChunk, (x + 1) kTileChunk), so neighbouring tiles, whose staged halos
-// overlap, meet in one L2 while the chunks stay spread over the XCDs.  The
-// last, partial group keeps the identity.  A bijection of [0, nblocks).
-constexpr int kTileChunk = 16;
-__device__ inline int xcd_tile(int b, int nblocks) {
-  constexpr int span = 8 * kTileChunk;
-  if (b >= nblocks / span * span) return b;
-  return b / span * span + (b % 8) * kTileChunk + (b / 8) % kTileChunk;
-}
-
 // Number of cell tiles (workgroups) of the tiled passes over grid g.
 inline long long tile_count(const GridDev& g) {
   if (!tile_shape_ok(g.tx, g.ty, g.tz)) throw std::logic_error("cell-tile shape out of range");
@@ -861,32 +500,38 @@ __device__ inline void tile_rows(const GridDev& g, int b, TileRows& T) {
   const int t = threadIdx.x;
   // row lengths in parallel: threads [0, nrows) staged rows (nrows <= 25),
   // [32, 32 + ntrows) target rows (ntrows <= 9)
+  int first = 0, len = 0;
   if (t < nrows) {
     const int row = ((sz0 + t / nyr) * g.ny + (sy0 + t % nyr)) * g.nx;
-    const int s = g.off[row + sx0];
-    T.start[t] = s;
-    T.base[t + 1] = g.off[row + sx1 + 1] - s;
+    first = g.off[row + sx0];
+    len = g.off[row + sx1 + 1] - first;
+    T.start[t] = first;
   } else if (t >= 32 && t < 32 + ntrows) {
     const int k = t - 32;
     const int row = ((cz0 + k / tyr) * g.ny + (cy0 + k % tyr)) * g.nx;
-    const int s = g.off[row + cx0];
-    T.tstart[k] = s;
-    T.tbase[k + 1] = g.off[row + cx1] - s;
+    first = g.off[row + cx0];
+    len = g.off[row + cx1] - first;
+    T.tstart[k] = first;
   }
-  __syncthreads();
-  if (t == 0) {
-    T.base[0] = 0;
-    for (int r = 0; r < nrows; ++r) {
-      const int len = T.base[r + 1];
-      T.base[r + 1] += T.base[r];
-      T.rend[r] = T.start[r] + len;
-      T.roff[r] = T.base[r] - T.start[r];
+  // prefix sums of the row lengths within wave 0 (staged rows) and its upper half (target rows)
+  if (t < 64) {
+    int v = len;
+    for (int off = 1; off < 32; off <<= 1) {
+      const int o = __shfl_up(v, off, 32);
+      if ((t & 31) >= off) v += o;
     }
-    T.nrows = nrows;
-  } else if (t == 64) {
-    T.tbase[0] = 0;
-    for (int k = 0; k < ntrows; ++k) T.tbase[k + 1] += T.tbase[k];
-    T.ntrows = ntrows;
+    if (t < nrows) {
+      T.base[t + 1] = v;
+      T.rend[t] = first + len;
+      T.roff[t] = v - len - first;
+    } else if (t >= 32 && t < 32 + ntrows) {
+      T.tbase[t - 32 + 1] = v;
+    }
+    if (t == 0) {
+      T.base[0] = T.tbase[0] = 0;
+      T.nrows = nrows;
+      T.ntrows = ntrows;
+    }
   }
   __syncthreads();
 }
@@ -958,130 +603,6 @@ __device__ inline int tile_round_fluid(const PV& pv, const NbrList& L, const Til
   return total;
 }
 
-template <int ST, bool CONT, bool THERMAL, bool KS>
-__global__ __launch_bounds__(kTileThreads) void k_forces_tiled(PV pv, GridDev g, SimParams P, NbrList L,
-                                                             DevState* st) {
-  __shared__ TileRows T;
-  __shared__ float4 s_x[kTileCap], s_rec[kTileCap], s_v[kTileCap], s_vt[kTileCap];
-  __shared__ float s_V[kTileCap];
-  __shared__ int s_work[kTileThreads], s_wave[kTileThreads / 64];
-  tile_rows(g, xcd_tile(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x)), T);
-  const int ntarget = T.tbase[T.ntrows];
-  if (ntarget == 0) return;  // uniform over the block
-  const int M = T.base[T.nrows];
-  const bool staged = M <= kTileCap;
-  const bool need_vt = forces_need_vt(P, CONT);
-  Maxima mx;
-  // Fluid targets packed onto consecutive threads (walls only write zeros):
-  // no lane idles through a pair loop for a wall.  The first round is
-  // packed before staging, so a tile of walls alone stages nothing.
-  auto none = [](auto&&) {};
-  auto other = [&](int i) { forces_particle<ST, CONT, THERMAL, KS>(pv, P, st, i, none, mx); };
-  const int nfl0 = tile_round_fluid(pv, L, T, ntarget, 0, s_work, s_wave, other);
-  if (nfl0 == 0 && ntarget <= kTileThreads) return;  // uniform over the block
-  if (staged) {
-    // Named slots, not arrays (arrays of them are not kept in registers).
-    struct Slot {
-      float4 x, r, v, t;
-      int ph;
-      float V;
-      float sig;
-    };
-    auto load = [&](int u) {
-      Slot q{};
-      const int s = threadIdx.x + u * kTileThreads;
-      if (s < M) {
-        const int j = tile_slot_index(T, s);
-        q.x = pv.s.x[j];
-        q.ph = pv.s.phase[j];
-        q.r = pv.t.nrec[j];
-        q.V = pv.t.vol[j];
-        const float4 v = pv.s.v[j];
-        float4 w = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (P.no_slip) w = pv.t.vw[j];
-        float4 t = v;
-        if (need_vt) t = pv.s.vt[j];
-        q.sig = 1.0f;
-        if (P.tvf) q.sig = pv.t.sigma[j];
-        q.v = q.ph == kWall ? w : v;
-        q.t = t;
-      }
-      return q;
-    };
-    auto store = [&](int u, const Slot q) {
-      const int s = threadIdx.x + u * kTileThreads;
-      if (s < M) {
-        s_x[s] = make_float4(q.x.x, q.x.y, q.x.z, __int_as_float(q.ph));
-        s_rec[s] = q.r;
-        // the velocity's free fourth component carries the neighbour's
-        // transport volume 1 / sigma, divided once per staged particle
-        s_v[s] = make_float4(q.v.x, q.v.y, q.v.z, P.tvf && is_fluid(q.ph) ? 1.0f / q.sig : 0.0f);
-        s_V[s] = q.V;
-        if (need_vt) s_vt[s] = q.t;
-      }
-    };
-    static_assert(kStageSlots == 5, "staging is written out for five slots per thread");
-    const Slot q0 = load(0), q1 = load(1), q2 = load(2), q3 = load(3), q4 = load(4);
-    store(0, q0);
-    store(1, q1);
-    store(2, q2);
-    store(3, q3);
-    store(4, q4);
-  }
-  __syncthreads();
-  for (int round = 0; round * kTileThreads < ntarget; ++round) {
-    const int nfl = round == 0 ? nfl0 : tile_round_fluid(pv, L, T, ntarget, round, s_work, s_wave, other);
-    if (static_cast<int>(threadIdx.x) >= nfl) continue;
-    const int i = s_work[threadIdx.x];
-    const int cnt = L.count[i];
-    if (staged) {
-      // Four neighbours at a time: their LDS records are read into registers
-      // (occupancy is set by LDS here, so registers are free) before the four
-      // pair bodies run, and the next four list entries are in flight.
-      auto from_lds = [&](auto&& f) {
-        RowCursor rc(T);
-        const int4* lp = list_chunks(L, i);
-        const int nq = (cnt + 3) >> 2;
-        int4 cur = nq > 0 ? lp[0] : make_int4(0, 0, 0, 0);
-        for (int q = 0; q < nq; ++q) {
-          int4 nxt = cur;
-          if (q + 1 < nq) nxt = lp[(q + 1) * kListGroup];
-          const int m = cnt - (q << 2);
-          const int js[4] = {cur.x, cur.y, cur.z, cur.w};
-          // the Akinci bodies hold more per-pair state: two records at a
-          // time (one with compensated sums) keep them within the register
-          // file (no scratch)
-          constexpr int kAhead = ST == 2 ? (KS ? 1 : 2) : 4;
-#pragma unroll
-          for (int h0 = 0; h0 < 4; h0 += kAhead) {
-            NbrData d[kAhead];
-#pragma unroll
-            for (int u = 0; u < kAhead; ++u) {
-              if (h0 + u < m) {
-                const int s = rc.slot(js[h0 + u]);
-                const float4 xs = s_x[s], rs = s_rec[s], vs = s_v[s];
-                float4 vts = vs;
-                if (need_vt) vts = s_vt[s];
-                d[u] = NbrData{xs, __float_as_int(xs.w), rs, vs, vts, s_V[s], vs.w};
-              }
-            }
-#pragma unroll
-            for (int u = 0; u < kAhead; ++u)
-              if (h0 + u < m) f(js[h0 + u], d[u]);
-          }
-          cur = nxt;
-        }
-      };
-      forces_particle<ST, CONT, THERMAL, KS>(pv, P, st, i, from_lds, mx);
-    } else {
-      auto gathered = [&](auto&& f) {
-        for_each_listed(L, i, cnt, [&](int j) { f(j, load_nbr(pv, P, j, need_vt)); });
-      };
-      forces_particle<ST, CONT, THERMAL, KS>(pv, P, st, i, gathered, mx);
-    }
-  }
-  publish_maxima(st, mx);
-}
 
 // ---------------------------------------------- interface, LDS-staged tiles
 // Same tiles and row tables as k_forces_tiled.  Staged per particle: x with
@@ -1370,41 +891,18 @@ void launch_heat_norm(DevState* st, const double* partials, int nb, bool active,
   k_heat_norm<<<1, 1024, 0, s>>>(st, partials, nb, active ? 1 : 0);
 }
 
-template <int ST, bool CONT, bool THERMAL, bool KS>
-static void forces_variant(const PV& pv, const GridDev& g, const SimParams& P, const NbrList& L, DevState* st, Count n,
-                           bool tiled, hipStream_t s) {
-  if (!L.valid) throw std::logic_error("forces pass: neighbour lists not built");
-  if (tiled) {
-    const long long tiles = tile_count(g);
-    if (tiles > 0x7fffffffLL) throw std::runtime_error("forces pass: too many cell tiles");
-    k_forces_tiled<ST, CONT, THERMAL, KS><<<static_cast<int>(tiles), kTileThreads, 0, s>>>(pv, g, P, L, st);
-  } else {
-    k_forces<ST, CONT, THERMAL, KS, false><<<blocks_for(n.ub > 0 ? n.ub : 1), kBlock, 0, s>>>(pv, g, P, L, st, n);
-  }
-  k_forces<ST, CONT, THERMAL, KS, true><<<blocks_for(n.ub > 0 ? n.ub : 1), kBlock, 0, s>>>(pv, g, P, L, st, n);
-}
-template <int ST, bool KS>
-static void forces_st(const PV& pv, const GridDev& g, const SimParams& P, const NbrList& L, DevState* st, Count n,
-                      bool continuity, bool thermal, bool tiled, hipStream_t s) {
-  if (continuity) {
-    if (thermal) forces_variant<ST, true, true, KS>(pv, g, P, L, st, n, tiled, s);
-    else forces_variant<ST, true, false, KS>(pv, g, P, L, st, n, tiled, s);
-  } else {
-    if (thermal) forces_variant<ST, false, true, KS>(pv, g, P, L, st, n, tiled, s);
-    else forces_variant<ST, false, false, KS>(pv, g, P, L, st, n, tiled, s);
-  }
-}
-template <bool KS>
-static void forces_ks(const PV& pv, const GridDev& g, const SimParams& P, const NbrList& L, DevState* st, Count n,
-                      bool csf_mode, bool akinci, bool continuity, bool thermal, bool tiled, hipStream_t s) {
-  if (akinci) forces_st<2, KS>(pv, g, P, L, st, n, continuity, thermal, tiled, s);
-  else if (csf_mode) forces_st<1, KS>(pv, g, P, L, st, n, continuity, thermal, tiled, s);
-  else forces_st<0, KS>(pv, g, P, L, st, n, continuity, thermal, tiled, s);
-}
+// Lanes per particle of the forces pass: four while the chip is not full
+// (shorter chains), two beyond (each lane of a group repeats the ordered
+// additions).  26 k particles 0.59 against 0.62 ms a step, 188 k particles
+// 0.89 against 0.87, 1.2 M 3.5 against 3.1.  `other` takes the other count.
+int forces_lanes(int n, bool other) { return (n < 120000) != other ? 4 : 2; }
+
 void launch_forces(const PV& pv, const GridDev& g, const SimParams& P, const NbrList& L, DevState* st, Count n,
-                   bool csf_mode, bool akinci, bool continuity, bool thermal, bool tiled, hipStream_t s) {
-  if (P.compensated) forces_ks<true>(pv, g, P, L, st, n, csf_mode, akinci, continuity, thermal, tiled, s);
-  else forces_ks<false>(pv, g, P, L, st, n, csf_mode, akinci, continuity, thermal, tiled, s);
+                   bool csf_mode, bool akinci, bool continuity, bool thermal, bool other_lanes, hipStream_t s) {
+  const int lanes = forces_lanes(n.ub, other_lanes);
+  if (akinci) launch_forces_akinci(pv, g, P, L, st, n, continuity, thermal, lanes, s);
+  else if (csf_mode) launch_forces_csf(pv, g, P, L, st, n, continuity, thermal, lanes, s);
+  else launch_forces_none(pv, g, P, L, st, n, continuity, thermal, lanes, s);
   k_publish_maxima<<<1, 1, 0, s>>>(st, P.has_vapor, P.sps);
 }
 void launch_probe(const PV& pv, const GridDev& g, const SimParams& P, const float* pts, float* out, int np,

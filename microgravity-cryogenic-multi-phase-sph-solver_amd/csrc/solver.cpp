@@ -227,6 +227,7 @@ struct cryo_solver {
   int set = 0;
   DevBuf<float4> a, ab, ns, vw, fw, mw, nrec;
   DevBuf<float> p, drho, dTdt, sigma, kappa, nu_t, alpha, wall_w, heat_w, out_m, out_h, w_norm, p_wv, rmin, vol;
+  DevBuf<PairRec> rec;  // neighbour records of the current rates evaluation
   // grid and scans
   DevBuf<uint32_t> keys_[2], vals_[2], tile_hist, row_total, split_flag, split_off, scan_sums, scan_total;
   DevBuf<int> cell_off;
@@ -238,10 +239,11 @@ struct cryo_solver {
   // Every particle [0, n) sits in the cell it was sorted into (no move or
   // append since the last sort): the cell-tile passes may be used.
   bool tiles_ok = false;
-  // Launch variants of the neighbour passes (results are the same bits either
-  // way): LDS-staged cell tiles or per-particle list gathers, for the
-  // interface and the forces pass.  autotune() times them.
-  bool tile_iface = true, tile_forces = true;
+  // Launch variants (results are the same bits either way): the forces pass
+  // with the number of lanes per particle its size rule gives or the other one,
+  // the interface pass over LDS-staged cell tiles or per-particle list gathers.
+  // autotune() times them.
+  bool tile_iface = true, rule_lanes = true;
   // cell-tile shape of the tiled passes (cells along x, y, z); any accepted
   // shape gives the same bits.  autotune_tiles() times candidates.
   int tile_shape[3] = {3, 3, 3};
@@ -410,7 +412,7 @@ struct cryo_solver {
                    rho_[k].get(), T_[k].get(), phase_[k].get(), flags_[k].get(), id_[k].get(), xlo_[k].get()};
     pv.t = Scratch{a.get(), ab.get(), ns.get(), vw.get(), fw.get(), mw.get(), p.get(), drho.get(), dTdt.get(),
                    sigma.get(), kappa.get(), nu_t.get(), alpha.get(), wall_w.get(), heat_w.get(), out_m.get(),
-                   out_h.get(), w_norm.get(), p_wv.get(), rmin.get(), nrec.get(), vol.get()};
+                   out_h.get(), w_norm.get(), p_wv.get(), rmin.get(), nrec.get(), vol.get(), rec.get()};
     pv.capacity = capacity;
     return pv;
   }
@@ -448,6 +450,7 @@ struct cryo_solver {
       if (cfg.compensated_sums) f(xlo_[k], k == set);
     }
     f(a, true); f(ab, true); f(ns, true); f(vw, true); f(fw, true); f(mw, true); f(nrec, false); f(vol, false);
+    f(rec, false);
     f(p, true); f(drho, true); f(dTdt, true); f(sigma, true); f(kappa, true); f(nu_t, true); f(alpha, true);
     f(wall_w, true); f(heat_w, true); f(out_m, true); f(out_h, true); f(w_norm, true); f(p_wv, true); f(rmin, true);
   }
@@ -550,6 +553,11 @@ struct cryo_solver {
     Q.eta_ll = harmonic(Q.mu[0], Q.mu[0]);
     Q.eta_lv = harmonic(Q.mu[0], Q.mu[1]);
     Q.eta_vv = harmonic(Q.mu[1], Q.mu[1]);
+    auto conductivity = [](float a, float b) { return 4.0f * a * b / (a + b); };
+    Q.k_ll = conductivity(Q.k[0], Q.k[0]);
+    Q.k_lv = conductivity(Q.k[0], Q.k[1]);
+    Q.k_vl = conductivity(Q.k[1], Q.k[0]);
+    Q.k_vv = conductivity(Q.k[1], Q.k[1]);
     Q.delta_sph = c.delta_sph;
     Q.density_mode = c.density_mode;
     Q.no_slip = c.no_slip ? 1 : 0;
@@ -603,6 +611,12 @@ struct cryo_solver {
     Q.heat_power = c.heater_power;
     Q.has_vapor = has_vapor ? 1 : 0;
     Q.compensated = c.compensated_sums ? 1 : 0;
+    // Range of the pair loops' fast arithmetic (recip_rn, sqrt_rn): the kernel
+    // gradient norm / h * q t^3 of a listed pair is 0 or at least norm / h * 2^-72,
+    // r2 + eta2 lies between 0.01 h^2 and 5 h^2.
+    Q.r2_fast = 1e-18f * h * h;
+    const float slope = Q.kernel.norm * Q.kernel.inv_h;
+    Q.fast = Q.r2_fast >= 0x1p-96f && Q.support2 <= 0x1p60f && slope >= 0x1p-26f && slope <= 0x1p90f ? 1 : 0;
     L = DtLimits{c.cfl, c.viscous_number, c.force_number, c.capillary_number, c.thermal_number,
                  c.dt_max, c.dt_min, c.fixed_dt};
   }
@@ -798,7 +812,7 @@ struct cryo_solver {
     }
     prof_begin(6);
     launch_forces(pv, gd, P, L, state.get(), nc, csf_mode, cfg.surface_tension == CRYO_ST_AKINCI,
-                  cfg.density_mode == CRYO_DENSITY_CONTINUITY, P.thermal != 0, tiles_ok && tile_forces, stream);
+                  cfg.density_mode == CRYO_DENSITY_CONTINUITY, P.thermal != 0, !rule_lanes, stream);
     prof_end(6);
     check_launch();
   }
@@ -1572,10 +1586,10 @@ struct cryo_solver {
   }
 
   // ----------------------------------------------------------- autotune
-  int launch_variant() const { return (tile_forces ? 0 : 1) | (tile_iface ? 0 : 2); }
+  int launch_variant() const { return (rule_lanes ? 0 : 1) | (tile_iface ? 0 : 2); }
   void set_launch_variant(int v) {
     if (v < 0 || v > 3) throw std::invalid_argument("launch variant must be 0..3");
-    tile_forces = (v & 1) == 0;
+    rule_lanes = (v & 1) == 0;
     tile_iface = (v & 2) == 0;
   }
   void set_tile_shape(int x, int y, int z) {

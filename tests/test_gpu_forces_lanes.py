@@ -1,0 +1,101 @@
+"""The forces pass with several lanes per particle, bit for bit against the FP32
+oracle where it can go wrong: both group sizes; particle counts that leave
+partial groups, waves and blocks; lists that overflow (the cell sweep); pairs
+outside the fast arithmetic's range (coincident and nearly coincident
+particles, an infinite temperature, fluid at rest), whose targets are done
+again with IEEE operations; tiny and large lengths that switch it off."""
+import numpy as np
+import pytest
+
+import cabi
+
+pytestmark = pytest.mark.gpu
+
+FIELDS = ("x", "v", "rho", "T", "p", "a", "ab", "fw", "mw", "drho", "dTdt", "kappa")
+
+
+def tank(scale=1.0, model="csf", seed=0):
+    fluid = cabi.hip_fluid_preset("LN2")
+    dx = float(np.float32(0.005 * scale))
+    kw = dict(dx=dx, gravity=(0, 0, -0.5), contact_angle_deg=20, velocity_scale=1.0)
+    if model == "column":
+        kw.update(surface_tension=0, thermal=0, phase_change=0, density_mode=1)
+    elif model == "akinci":
+        kw.update(surface_tension=2, thermal=0, phase_change=0, contact_angle_deg=60)
+    elif model == "sps":
+        kw.update(surface_tension=0, thermal=0, phase_change=0, density_mode=1, sps_turbulence=1)
+    cfg = cabi.default_config(**kw)
+    s = 0.04 * scale
+    ps = cabi.hip_build_tank_particles(cabi.box(s, s, s), fluid, dx, cabi.default_fill(
+        include_vapor=1 if model == "csf" else 0, T_liquid=fluid.T_sat + 1.0))
+    rng = np.random.default_rng(seed)
+    fl = ps.phase != cabi.WALL
+    ps.x[fl] += (0.05 * dx * rng.uniform(-1, 1, (int(fl.sum()), 3))).astype(np.float32)
+    ps.v[fl] = rng.normal(0, 0.05, (int(fl.sum()), 3)).astype(np.float32)
+    return fluid, cfg, ps, dx
+
+
+def take(ps, keep):
+    return cabi.ParticleSet(ps.x[keep], ps.v[keep], ps.nrm[keep], ps.m[keep], ps.rho[keep], ps.T[keep], ps.phase[keep],
+                            ps.flags[keep], None)
+
+
+def check(fluid, cfg, ps, dx, variant, steps=2):
+    lo, hi = ps.x.min(0) - 4 * dx, ps.x.max(0) + 4 * dx
+    gpu, cpu = cabi.HipSolver(cfg, fluid), cabi.CpuSolver("orc", cfg, fluid, 32)
+    gpu.set_launch_variant(variant)
+    for s in (gpu, cpu):
+        s.set_particles(ps, lo, hi)
+        s.next_dt()
+    for k in range(2):
+        for f in FIELDS:
+            a, b = gpu.field(f), cpu.field(f)
+            assert np.array_equal(a, b, equal_nan=True), (f, k, int((a != b).sum()))
+        if k == 0 and steps:
+            gpu.run_steps(steps)
+            cpu.run_steps(steps)
+
+
+@pytest.mark.parametrize("variant", [0, 1])
+@pytest.mark.parametrize("model", ["csf", "column", "akinci", "sps"])
+@pytest.mark.parametrize("drop", [0, 1, 63])
+def test_group_sizes_and_remainders(model, variant, drop):
+    fluid, cfg, ps, dx = tank(model=model)
+    n = len(ps) // 64 * 64 + 1 - drop
+    print("lanes", model, variant, n, flush=True)
+    walls = np.flatnonzero(ps.phase == cabi.WALL)
+    keep = np.ones(len(ps), bool)
+    keep[walls[:len(ps) - n]] = False
+    check(fluid, cfg, take(ps, keep), dx, variant)
+
+
+@pytest.mark.parametrize("variant", [0, 1])
+@pytest.mark.parametrize("case", ["crowd", "coincident", "close", "hot", "rest"])
+def test_particles_outside_the_fast_range(case, variant):
+    fluid, cfg, ps, dx = tank()
+    fl = np.flatnonzero(ps.phase == cabi.LIQUID)
+    steps = 2
+    print("lanes", case, variant, flush=True)
+    if case == "crowd":  # more than 96 neighbours each
+        ps.x[fl[:160]] = ps.x[fl[80]] + (0.4 * dx * np.random.default_rng(1).uniform(-1, 1, (160, 3))).astype(np.float32)
+        assert len(fl) >= 160
+        steps = 0
+    elif case == "coincident":
+        ps.x[fl[10]] = ps.x[fl[11]]
+        steps = 0
+    elif case == "close":
+        ps.x[fl[10]] = np.nextafter(ps.x[fl[11]], np.float32(1))
+        steps = 0
+    elif case == "hot":
+        ps.T[fl[20]] = np.float32(np.inf)
+        steps = 0
+    else:
+        ps.v[:] = 0
+    check(fluid, cfg, ps, dx, variant, steps)
+
+
+@pytest.mark.parametrize("scale", [2e-4, 1e6])
+def test_lengths_beyond_the_fast_range(scale):
+    fluid, cfg, ps, dx = tank(scale=scale, model="column")
+    print("lanes scale", scale, flush=True)
+    check(fluid, cfg, ps, dx, 0, steps=1)
