@@ -11,6 +11,7 @@
 // Every accumulator adds its neighbours in the reference order (ascending
 // sorted index), with the reference's per-pair expressions, so each field is
 // the same float the reference computes (given equal inputs).
+#include <algorithm>
 #include <stdexcept>
 
 #include "pair_lanes.hpp"
@@ -33,52 +34,29 @@ __device__ inline void block_sum_store(double v, double* out) {
   }
 }
 
-// ------------------------------------------------------- density + EOS
-// Also builds the step's neighbour lists from the same (cell-culled) sweep.
+// W at squared distance r2 (below r2_fast it is its value at 0 to the last bit).
+__device__ inline float kernel_at(const SimParams& P, float r2) {
+  return kW(P.kernel, P.fast ? sqrt_rn(r2 < P.r2_fast ? P.r2_fast : r2) : sqrtf(r2));
+}
+
+// Density, pressure and neighbour record of particle i from its kernel sum and
+// squared nearest distance.
 template <bool KS>
-__global__ __launch_bounds__(kBlock) void k_density(PV pv, GridDev g, SimParams P, NbrList L, Count nc) {
-  const int n = nc.get();
-  const int i = gtid();
-  if (i >= n) return;
+__device__ inline void density_finish(const PV& pv, const SimParams& P, int i, const Acc<KS>& sum, float r2min) {
   const uint8_t ph = pv.s.phase[i];
   const V3 xi = ld3(pv.s.x[i]);
-  ListWriter lw(L, i);
   if (!is_fluid(ph)) {
     pv.t.sigma[i] = 1.0f / P.vol0;
     pv.t.rmin[i] = P.kernel.support;
-    // wall targets only ever need their fluid neighbours: none without a fluid
-    // particle in the 27 cells
-    if (ph == kWall && cells_any(g, xi, kCellFluid)) {
-      for_each_cand_xph(g, xi, P.kernel.support, pv.s.x, pv.s.phase, [&](int j, float4 xj, uint8_t phj) {
-        if (norm2(xi - ld3(xj)) >= P.support2) return;
-        if (!is_fluid(phj)) return;
-        lw.push(j);
-      });
-    }
-    L.count[i] = lw.finish();
     if (ph != kWall) {  // dead, not yet dropped: what the last evaluation gave it, at its present phase and velocity
       const float4 v = pv.s.v[i];
-      PairRec& r = pv.t.rec[i];
-      r.x = make_float4(xi.x, xi.y, xi.z, __int_as_float(ph));
-      r.v = make_float4(v.x, v.y, v.z, r.v.w);
-      r.t = st3(ld3(pv.s.vt[i]));
+      PairRec& rec = pv.t.rec[i];
+      rec.x = make_float4(xi.x, xi.y, xi.z, __int_as_float(ph));
+      rec.v = make_float4(v.x, v.y, v.z, rec.v.w);
+      rec.t = st3(ld3(pv.s.vt[i]));
     }
     return;
   }
-  Acc<KS> sum;
-  float r2min = P.support2;
-  const V3 li = pos_lo<KS>(pv.s.xlo, i);
-  for_each_cand_x(g, xi, P.kernel.support, pv.s.x, [&](int j, float4 xj) {
-    // neighbourhood by the float positions (the lists of every later pass);
-    // in the precision form the kernel takes the double-float distance
-    const float r2h = norm2(xi - ld3(xj));
-    if (r2h >= P.support2) return;
-    const float r2 = KS ? norm2(pos_diff<KS>(xi, li, ld3(xj), pv.s.xlo, j)) : r2h;
-    sum += kW(P.kernel, sqrtf(r2));
-    if (j != i && r2 < r2min) r2min = r2;
-    lw.push(j);
-  });
-  L.count[i] = lw.finish();
   pv.t.sigma[i] = float(sum);
   pv.t.rmin[i] = sqrtf(r2min);
   float rho = pv.s.rho[i];
@@ -109,6 +87,206 @@ __global__ __launch_bounds__(kBlock) void k_density(PV pv, GridDev g, SimParams 
   const float4 v = pv.s.v[i], vt = pv.s.vt[i];
   pv.t.rec[i] = PairRec{make_float4(xi.x, xi.y, xi.z, __int_as_float(ph)), q, make_float4(v.x, v.y, v.z, V),
                         make_float4(vt.x, vt.y, vt.z, P.tvf ? 1.0f / float(sum) : 0.0f)};
+}
+
+// ------------------------------------------------------- density + EOS
+// Also builds the step's neighbour lists from the same (cell-culled) sweep.
+// A row of 16 lanes takes one particle: its lanes 0..8 look the nine cell rows
+// up side by side, then the lanes test 16 candidates at a time; the hits, in
+// candidate order, go to the list and their squared distances to LDS, from
+// where 16 kernel values at a time are evaluated and added in order.  (One
+// thread per particle ran a chain of about 350 candidate tests, and the kernel
+// evaluation for every one that any lane of the wave hit: 156 us at any size
+// up to 100 k particles; now 28 us at 26 k.)  A block takes 16 consecutive
+// particles and writes their results coalesced.
+constexpr int kDensLanes = 16;
+constexpr int kDensRing = 128;  // hits of one particle waiting for their kernel values
+template <bool KS>
+__global__ __launch_bounds__(kBlock) void k_density(PV pv, GridDev g, SimParams P, NbrList L, Count nc) {
+  constexpr int kGroups = kBlock / kDensLanes, kSpan = kGroups;
+  using Ln = Lanes<kDensLanes>;
+  __shared__ int2 s_row[kGroups][9];           // one past the row's last candidate number; sorted index - number
+  __shared__ float s_r2[kGroups][kDensRing];
+  __shared__ float s_sum[kSpan], s_low[kSpan], s_min[kSpan];
+  __shared__ int s_count[kSpan];
+  const int n = nc.get();
+  const int base = xcd_span(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x)) * kSpan;
+  if (base >= n) return;  // uniform over the block
+  const int grp = static_cast<int>(threadIdx.x) / kDensLanes, l = threadIdx.x % kDensLanes;
+  const int lane = threadIdx.x & 63;
+  const int row0 = lane & ~(kDensLanes - 1);
+  const float4* __restrict__ xs = pv.s.x;
+  const int me = base + grp;
+  const bool here = me < n;
+  const uint8_t ph = here ? pv.s.phase[me] : kDead;
+  const bool fluid = is_fluid(ph);
+  const V3 xi = here ? ld3(xs[me]) : V3{0, 0, 0};
+  V3 li{0, 0, 0};
+  if (KS && fluid) li = ld3(pv.s.xlo[me]);
+  // the nine rows of the 27 cells (for_each_cand), one per lane
+  const float ux = (xi.x - g.ox) * g.inv_cell, uy = (xi.y - g.oy) * g.inv_cell, uz = (xi.z - g.oz) * g.inv_cell;
+  const int cx = clampv(static_cast<int>(floorf(ux)), 0, g.nx - 1);
+  const int cy = clampv(static_cast<int>(floorf(uy)), 0, g.ny - 1);
+  const int cz = clampv(static_cast<int>(floorf(uz)), 0, g.nz - 1);
+  const int dz = l / 3 - 1, dy = l % 3 - 1;
+  const int z = cz + dz, y = cy + dy;
+  int first = 0, len = 0;
+  bool near_fluid = false;
+  if (here && ph != kDead && l < 9 && z >= 0 && z < g.nz && y >= 0 && y < g.ny) {
+    const int row = (z * g.ny + y) * g.nx;
+    const float fx = ux - static_cast<float>(cx), fy = uy - static_cast<float>(cy), fz = uz - static_cast<float>(cz);
+    const float rc = P.kernel.support * g.inv_cell + g.cull_pad;
+    const float rr = rc * rc;
+    const float gz = dz < 0 ? fz : (dz > 0 ? 1.0f - fz : 0.0f);
+    const float gy = dy < 0 ? fy : (dy > 0 ? 1.0f - fy : 0.0f);
+    const float gyz = gy * gy + gz * gz;
+    if (!(gyz >= rr)) {
+      const int x0 = (cx > 0 && gyz + fx * fx < rr) ? cx - 1 : cx;
+      const int x1 = (cx < g.nx - 1 && gyz + (1.0f - fx) * (1.0f - fx) < rr) ? cx + 1 : cx;
+      first = g.off[row + x0];
+      len = g.off[row + x1 + 1] - first;
+    }
+    if (!fluid) {
+      const int x0 = cx > 0 ? cx - 1 : 0, x1 = cx < g.nx - 1 ? cx + 1 : cx;
+      int any = 0;
+      for (int x = x0; x <= x1; ++x) any |= g.flags[row + x];
+      near_fluid = (any & kCellFluid) != 0;
+    }
+  }
+  // wall targets only ever need their fluid neighbours: none without a fluid
+  // particle in the 27 cells
+  const unsigned rows_fluid = static_cast<unsigned>(__ballot(near_fluid) >> row0) & 0xffffu;
+  if (!fluid && rows_fluid == 0) len = 0;
+  int end = len;
+#pragma unroll
+  for (int off = 1; off < kDensLanes; off <<= 1) {
+    const int o = __shfl_up(end, off, kDensLanes);
+    if (l >= off) end += o;
+  }
+  if (l < 9) s_row[grp][l] = make_int2(end, first - (end - len));
+  const int total = __shfl(end, kDensLanes - 1, kDensLanes);
+  wave_lds_fence();
+  Acc<KS> sum;
+  float r2min = P.support2;
+  int c = 0, done = 0;
+  int* out = reinterpret_cast<int*>(list_chunks(L, here ? me : 0));
+  // adds the kernel values of hits [done, done + 16) below c
+  auto drain = [&]() {
+    const int k = done + l;
+    const float r2 = s_r2[grp][k & (kDensRing - 1)];
+    float w = 0.0f;
+    if (k < c) w = kernel_at(P, r2);
+    unrolled<kDensLanes>([&](auto kc) { sum += Ln::template from<decltype(kc)::value>(w); });
+    done += kDensLanes;
+  };
+  int2 row = s_row[grp][0];
+  int r = 0;
+  auto index = [&](int v) {  // sorted index of candidate v; the particle itself past the end
+    if (v >= total) return here ? me : 0;
+    while (v >= row.x) row = s_row[grp][++r];
+    return v + row.y;
+  };
+  int j = index(l);
+  float4 x = xs[j];
+  uint8_t q = kLiquid;
+  if (!fluid) q = pv.s.phase[j];
+  for (int v = l; __any(v - l < total); v += kDensLanes) {
+    const float4 xj = take(x);
+    const int jc = j;
+    const bool usable = v < total && (fluid || is_fluid(q));
+    if (v - l + kDensLanes < total) {
+      j = index(v + kDensLanes);
+      x = xs[j];
+      if (!fluid) q = pv.s.phase[j];
+    }
+    // neighbourhood by the float positions (the lists of every later pass);
+    // in the precision form the kernel takes the double-float distance
+    const float r2h = norm2(xi - ld3(xj));
+    const bool hit = usable && !(r2h >= P.support2);
+    const unsigned hits = static_cast<unsigned>(__ballot(hit) >> row0) & 0xffffu;
+    if (hit) {
+      const int e = c + __popc(hits & ((1u << l) - 1u));
+      if (e < L.K) out[(e >> 2) * (4 * kListGroup) + (e & 3)] = jc;
+      if (fluid) {
+        const float r2 = KS ? norm2(pos_diff<KS>(xi, li, ld3(xj), pv.s.xlo, jc)) : r2h;
+        if (jc != me && r2 < r2min) r2min = r2;
+        s_r2[grp][e & (kDensRing - 1)] = r2;
+      }
+    }
+    c += __popc(hits);
+    if (__any(fluid && c - done > kDensRing - kDensLanes)) {
+      wave_lds_fence();
+      if (fluid)
+        while (c - done >= kDensLanes) drain();
+    }
+  }
+  wave_lds_fence();
+  if (fluid)
+    while (done < c) drain();
+  for (int off = kDensLanes / 2; off > 0; off >>= 1) {
+    const float o = __shfl_xor(r2min, off, kDensLanes);
+    r2min = o < r2min ? o : r2min;
+  }
+  if (l == 0) {
+    if constexpr (KS) {
+      s_sum[grp] = sum.s;
+      s_low[grp] = sum.c;
+    } else {
+      s_sum[grp] = sum;
+    }
+    s_min[grp] = r2min;
+    s_count[grp] = c <= L.K ? c : -1;
+  }
+  __syncthreads();
+  const int slot = threadIdx.x;
+  const int i = base + slot;
+  if (slot >= kSpan || i >= n) return;
+  L.count[i] = s_count[slot];
+  Acc<KS> whole;
+  whole.s = s_sum[slot];
+  if constexpr (KS) whole.c = s_low[slot];
+  density_finish<KS>(pv, P, i, whole, s_min[slot]);
+}
+
+// One thread per particle: what very large sets take (from kDensWide on, where
+// every SIMD is full either way and the shorter chains of the row of lanes
+// above no longer pay for its bookkeeping: 2.2 M particles 1120 us with it).
+constexpr int kDensWide = 700000;
+template <bool KS>
+__global__ __launch_bounds__(kBlock) void k_density_wide(PV pv, GridDev g, SimParams P, NbrList L, Count nc) {
+  const int n = nc.get();
+  const int i = gtid();
+  if (i >= n) return;
+  const uint8_t ph = pv.s.phase[i];
+  const V3 xi = ld3(pv.s.x[i]);
+  ListWriter lw(L, i);
+  Acc<KS> sum;
+  float r2min = P.support2;
+  if (!is_fluid(ph)) {
+    // wall targets only ever need their fluid neighbours: none without a fluid
+    // particle in the 27 cells
+    if (ph == kWall && cells_any(g, xi, kCellFluid)) {
+      for_each_cand_xph(g, xi, P.kernel.support, pv.s.x, pv.s.phase, [&](int j, float4 xj, uint8_t phj) {
+        if (norm2(xi - ld3(xj)) >= P.support2) return;
+        if (!is_fluid(phj)) return;
+        lw.push(j);
+      });
+    }
+  } else {
+    const V3 li = pos_lo<KS>(pv.s.xlo, i);
+    for_each_cand_x(g, xi, P.kernel.support, pv.s.x, [&](int j, float4 xj) {
+      // neighbourhood by the float positions (the lists of every later pass);
+      // in the precision form the kernel takes the double-float distance
+      const float r2h = norm2(xi - ld3(xj));
+      if (r2h >= P.support2) return;
+      const float r2 = KS ? norm2(pos_diff<KS>(xi, li, ld3(xj), pv.s.xlo, j)) : r2h;
+      sum += kernel_at(P, r2);
+      if (j != i && r2 < r2min) r2min = r2;
+      lw.push(j);
+    });
+  }
+  L.count[i] = lw.finish();
+  density_finish<KS>(pv, P, i, sum, r2min);
 }
 
 // SPH_kernels.cu:36-54 (start-up only).
@@ -239,6 +417,52 @@ __device__ inline IfaceNbr load_iface_nbr(const PV& pv, const SimParams& P, int 
   return d;
 }
 
+// The interface fields of fluid particle i from its sums.
+__device__ inline void interface_finish(const PV& pv, const SimParams& P, int i, uint8_t ph, int csf_mode, V3 gradc,
+                                        V3 wall_n, V3 akn, V3 gradphi, float s_all, float s_other, float ww,
+                                        float hw) {
+  pv.t.alpha[i] = s_all > 0.0f ? s_other / s_all : 0.0f;
+  pv.t.wall_w[i] = ww;
+  pv.t.heat_w[i] = hw;
+  if (P.st_model == 2) {
+    pv.s.nrm[i] = st3(ph == kLiquid ? akn * (-P.kernel.h) : V3{0, 0, 0});
+  } else {
+    const float gmag = norm(gradc);
+    V3 vwi{0, 0, 0};
+    if (P.wetting != 0 && ww > 0.0f && gmag > P.normal_eps && norm2(wall_n) > 0.0f) {
+      const V3 nw = normalized(wall_n);
+      const V3 nh = gradc / gmag;
+      const V3 tan_in = nh - nw * dot(nh, nw);
+      const float tm = norm(tan_in);
+      if (tm > 1e-6f) {
+        const float cos_d = -dot(nh, nw);
+        const float delta_w = 2.0f * norm(gradphi);
+        const float coeff = 2.0f * P.sigma / (P.rho0[0] + P.rho0[1]);
+        vwi = tan_in * (-(P.cos_theta - cos_d) * coeff * gmag * delta_w / tm);
+      }
+    }
+    pv.t.vw[i] = st3(vwi);
+    if (P.wetting != 1 && ww > 0.0f && gmag > P.normal_eps) {
+      const V3 nw = normalized(wall_n);
+      const V3 nh = gradc / gmag;
+      V3 t = nh - nw * dot(nh, nw);
+      const float tmag = norm(t);
+      if (norm2(nw) > 0.0f && tmag > 1e-6f) {
+        t = t / tmag;
+        const V3 target = nw * (-P.cos_theta) + t * P.sin_theta;
+        const float beta = clampv(ww / P.wall_adh_w, 0.0f, 1.0f);
+        const V3 blended = normalized(nh * (1.0f - beta) + target * beta);
+        gradc = blended * gmag;
+      }
+    }
+    pv.s.nrm[i] = st3(gradc);
+    if (csf_mode && !P.csf_smooth) {
+      const float gm = norm(gradc);
+      pv.t.ns[i] = st3(!(gm > P.normal_eps) ? V3{0, 0, 0} : gradc / gm);
+    }
+  }
+}
+
 // compute_interface_fields (surface_tension.cu:5-85) + SPS (navier_stokes.cu:
 // 71-119) + normals without smoothing (surface_tension.cu:87-118) for particle
 // i; returns its heat weight (0 unless fluid).  visit(f): f(j, IfaceNbr) over
@@ -292,8 +516,6 @@ __device__ inline float interface_particle(const PV& pv, const SimParams& P, int
     agradc += gw * (Vj * (cj - ci));
     if (phj == kLiquid) aakn += gw * Vj;
   });
-  V3 gradc = agradc;
-  const V3 wall_n = awall_n, akn = aakn, gradphi = agradphi;
   const float s_all = as_all, s_other = as_other, ww = aww, hw = ahw;
   if (SPS) {
     float ss = 0.0f;
@@ -306,46 +528,7 @@ __device__ inline float interface_particle(const PV& pv, const SimParams& P, int
     const float l = P.smag_cs * P.dx;
     pv.t.nu_t[i] = l * l * smag;
   }
-  pv.t.alpha[i] = s_all > 0.0f ? s_other / s_all : 0.0f;
-  pv.t.wall_w[i] = ww;
-  pv.t.heat_w[i] = hw;
-  if (P.st_model == 2) {
-    pv.s.nrm[i] = st3(ph == kLiquid ? akn * (-P.kernel.h) : V3{0, 0, 0});
-  } else {
-    const float gmag = norm(gradc);
-    V3 vwi{0, 0, 0};
-    if (P.wetting != 0 && ww > 0.0f && gmag > P.normal_eps && norm2(wall_n) > 0.0f) {
-      const V3 nw = normalized(wall_n);
-      const V3 nh = gradc / gmag;
-      const V3 tan_in = nh - nw * dot(nh, nw);
-      const float tm = norm(tan_in);
-      if (tm > 1e-6f) {
-        const float cos_d = -dot(nh, nw);
-        const float delta_w = 2.0f * norm(gradphi);
-        const float coeff = 2.0f * P.sigma / (P.rho0[0] + P.rho0[1]);
-        vwi = tan_in * (-(P.cos_theta - cos_d) * coeff * gmag * delta_w / tm);
-      }
-    }
-    pv.t.vw[i] = st3(vwi);
-    if (P.wetting != 1 && ww > 0.0f && gmag > P.normal_eps) {
-      const V3 nw = normalized(wall_n);
-      const V3 nh = gradc / gmag;
-      V3 t = nh - nw * dot(nh, nw);
-      const float tmag = norm(t);
-      if (norm2(nw) > 0.0f && tmag > 1e-6f) {
-        t = t / tmag;
-        const V3 target = nw * (-P.cos_theta) + t * P.sin_theta;
-        const float beta = clampv(ww / P.wall_adh_w, 0.0f, 1.0f);
-        const V3 blended = normalized(nh * (1.0f - beta) + target * beta);
-        gradc = blended * gmag;
-      }
-    }
-    pv.s.nrm[i] = st3(gradc);
-    if (csf_mode && !P.csf_smooth) {
-      const float gm = norm(gradc);
-      pv.t.ns[i] = st3(!(gm > P.normal_eps) ? V3{0, 0, 0} : gradc / gm);
-    }
-  }
+  interface_finish(pv, P, i, ph, csf_mode, agradc, awall_n, aakn, agradphi, s_all, s_other, ww, hw);
   return hw;
 }
 
@@ -356,8 +539,86 @@ __device__ inline float interface_particle(const PV& pv, const SimParams& P, int
 // outputs of an empty sum directly.  Without vapour at all, a wall within 2h
 // of a liquid particle has colour alpha_w = 1 and so adds zeros too: only wall
 // neighbours are summed.  Bitwise the full pass's results (adding a zero to a
-// running sum that starts at +0 never changes it).  Resets the dt maxima and
-// writes the heat partials as k_interface does.
+// running sum that starts at +0 never changes it).  Resets the dt maxima.
+// A row of 16 lanes per particle that has a wall or the other phase nearby, up
+// to kInterfaceLanes particles: 26 k 66 -> 26 us, 4 k 77 -> 15; 188 k would
+// take 102 us with it, 88 with one thread per particle (13 ordered sums, each
+// repeated by 16 lanes).
+constexpr int kInterfaceLanes = 100000;
+template <bool KS, int G>
+__global__ __launch_bounds__(kBlock) void k_interface_lanes(PV pv, GridDev g, SimParams P, NbrList L, DevState* st,
+                                                            Count nc, int csf_mode, int span) {
+  const int n = nc.get();
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    for (int k = 0; k < 5; ++k) st->max_bits[k] = 0u;
+  }
+  const int base = xcd_span(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x)) * span;
+  if (base >= n) return;  // uniform over the block
+  auto select = [&](int i) {
+    const uint8_t ph = pv.s.phase[i];
+    if (!is_fluid(ph)) return false;
+    if (cells_any(g, ld3(pv.s.x[i]), kCellWall | (ph == kLiquid ? kCellVapor : kCellLiquid))) return true;
+    pv.t.alpha[i] = 0.0f;
+    pv.t.wall_w[i] = 0.0f;
+    pv.t.heat_w[i] = 0.0f;
+    pv.t.vw[i] = st3(V3{0, 0, 0});
+    pv.s.nrm[i] = st3(V3{0, 0, 0});
+    if (csf_mode && !P.csf_smooth) pv.t.ns[i] = st3(V3{0, 0, 0});
+    return false;
+  };
+  for_each_group<G>(base, span, n, select, [&](int i, int sub) {
+    const uint8_t ph = pv.s.phase[i];
+    const V3 xi = ld3(pv.s.x[i]);
+    const V3 li = pos_lo<KS>(pv.s.xlo, i);
+    const float ci = ph == kLiquid ? 1.0f : 0.0f;
+    // colour gradient, wall normal, wall gradient (x, y, z each), alpha's
+    // denominator and numerator, wall and heater weights
+    Acc<KS> a[13];
+    lane_sums<G>(L, g, i, xi, sub, a, [&](int j, float (&t)[13]) {
+      // the gathers in flight together (a wall's normal and colour only for
+      // walls: this pass writes the fluid ones)
+      const int phj = pv.s.phase[j], flags = pv.s.flags[j];
+      const float4 xj = pv.s.x[j];
+      const float Vj = pv.t.vol[j];
+      settle(phj, flags, xj.x, xj.y, xj.z, Vj);
+      if (!P.has_vapor && phj != kWall) return;
+      const V3 rij = pos_diff<KS>(xi, li, ld3(xj), pv.s.xlo, j);
+      const float r2 = norm2(rij);
+      if (r2 >= P.support2) return;
+      const float r = sqrtf(r2);
+      const float w = kW(P.kernel, r);
+      const V3 gw = kgradW(P.kernel, rij, r);
+      if (phj == kWall) {
+        const float vw = P.vol0 * w;
+        t[11] = vw;
+        if (flags & kHeated) t[12] = vw;
+        const V3 nw = ld3(pv.s.nrm[j]) * vw;
+        t[3] = nw.x, t[4] = nw.y, t[5] = nw.z;
+        const V3 gp = gw * P.vol0;
+        t[6] = gp.x, t[7] = gp.y, t[8] = gp.z;
+        if (P.wall_colour) {
+          const V3 gc = gw * (P.vol0 * (pv.t.alpha[j] - ci));
+          t[0] = gc.x, t[1] = gc.y, t[2] = gc.z;
+        }
+        return;
+      }
+      t[9] = Vj * w;
+      if (phj != ph) t[10] = Vj * w;
+      if (j == i) return;
+      const float cj = phj == kLiquid ? 1.0f : 0.0f;
+      const V3 gc = gw * (Vj * (cj - ci));
+      t[0] = gc.x, t[1] = gc.y, t[2] = gc.z;
+    });
+    if (sub == 0)
+      interface_finish(pv, P, i, ph, csf_mode, V3{float(a[0]), float(a[1]), float(a[2])},
+                       V3{float(a[3]), float(a[4]), float(a[5])}, V3{0, 0, 0},
+                       V3{float(a[6]), float(a[7]), float(a[8])}, float(a[9]), float(a[10]), float(a[11]),
+                       float(a[12]));
+  });
+}
+
+// The same with one thread per particle (many particles); also writes the heat
+// partials.
 template <bool KS>
 __global__ __launch_bounds__(kBlock) void k_interface_sparse(PV pv, GridDev g, SimParams P, NbrList L, DevState* st,
                                                             Count nc, int csf_mode, double* heat_partials) {
@@ -834,8 +1095,14 @@ __global__ __launch_bounds__(kBlock) void k_shift_apply(PV pv, Count nc) {
 
 void launch_density(const PV& pv, const GridDev& g, const SimParams& P, const NbrList& L, Count n, hipStream_t s) {
   if (n.ub <= 0) return;
-  if (P.compensated) k_density<true><<<blocks_for(n.ub), kBlock, 0, s>>>(pv, g, P, L, n);
-  else k_density<false><<<blocks_for(n.ub), kBlock, 0, s>>>(pv, g, P, L, n);
+  if (n.ub >= kDensWide) {
+    if (P.compensated) k_density_wide<true><<<blocks_for(n.ub), kBlock, 0, s>>>(pv, g, P, L, n);
+    else k_density_wide<false><<<blocks_for(n.ub), kBlock, 0, s>>>(pv, g, P, L, n);
+    return;
+  }
+  const int nb = blocks_for(static_cast<long long>(n.ub) * kDensLanes);
+  if (P.compensated) k_density<true><<<nb, kBlock, 0, s>>>(pv, g, P, L, n);
+  else k_density<false><<<nb, kBlock, 0, s>>>(pv, g, P, L, n);
 }
 void launch_normalize_masses(const PV& pv, const GridDev& g, const SimParams& P, int n, hipStream_t s) {
   if (n <= 0) return;
@@ -867,8 +1134,15 @@ int launch_interface(const PV& pv, const GridDev& g, const SimParams& P, const N
   const int nb = blocks_for(n.ub > 0 ? n.ub : 1);
   const int cm = csf_mode ? 1 : 0;
   if (P.st_model != 2 && !P.sps && L.valid && g.flags) {
-    if (P.compensated) k_interface_sparse<true><<<nb, kBlock, 0, s>>>(pv, g, P, L, st, n, cm, heat_partials);
-    else k_interface_sparse<false><<<nb, kBlock, 0, s>>>(pv, g, P, L, st, n, cm, heat_partials);
+    if (n.ub < kInterfaceLanes) {
+      const int span = lane_span(n.ub), sb = (std::max(n.ub, 1) + span - 1) / span;
+      if (P.compensated) k_interface_lanes<true, 16><<<sb, kBlock, 0, s>>>(pv, g, P, L, st, n, cm, span);
+      else k_interface_lanes<false, 16><<<sb, kBlock, 0, s>>>(pv, g, P, L, st, n, cm, span);
+      if (heat_partials) k_heat_partials<<<nb, kBlock, 0, s>>>(pv, n, heat_partials);
+    } else {
+      if (P.compensated) k_interface_sparse<true><<<nb, kBlock, 0, s>>>(pv, g, P, L, st, n, cm, heat_partials);
+      else k_interface_sparse<false><<<nb, kBlock, 0, s>>>(pv, g, P, L, st, n, cm, heat_partials);
+    }
     return nb;
   }
   tiled = tiled && L.valid;

@@ -7,15 +7,13 @@
 // ullage state stay in a device-resident DevState, and every FP64 sum is a
 // fixed-order two-level reduction (block partials, then one ordered block),
 // so runs are bitwise reproducible.
-#include "kernels.hpp"
+#include <algorithm>
+
+#include "pair_lanes.hpp"
 
 namespace cryo {
 
 namespace {
-
-constexpr int kBlock = 256;
-__device__ inline int gtid() { return static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x); }
-inline int blocks_for(long long n) { return static_cast<int>((n + kBlock - 1) / kBlock); }
 
 template <int NQ>
 __device__ inline void block_sums_store(double (&v)[NQ], double* partials, int stride) {
@@ -243,6 +241,70 @@ __global__ __launch_bounds__(kBlock) void k_pc_normalize(PV pv, GridDev g, SimPa
   block_sums_store<3>(acc, partials, stride);
 }
 
+// The same for fewer particles: a row of 16 lanes per source, then the partials
+// (k_pc_partials).
+template <bool KS, int G>
+__global__ __launch_bounds__(kBlock) void k_pc_normalize_lanes(PV pv, GridDev g, SimParams P, NbrList L, Count nc,
+                                                              int span) {
+  const int n = nc.get();
+  const int base = xcd_span(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x)) * span;
+  if (base >= n) return;  // uniform over the block
+  auto select = [&](int i) { return (pv.s.flags[i] & kSource) != 0; };
+  for_each_group<G>(base, span, n, select, [&](int i, int sub) {
+    const uint8_t fl = pv.s.flags[i];
+    const uint8_t target = (fl & kTargetVapor) ? kVapor : kLiquid;
+    const V3 xi = ld3(pv.s.x[i]);
+    const V3 li = pos_lo<KS>(pv.s.xlo, i);
+    Acc<KS> a[1];
+    float wr_max = 0.0f;
+    lane_sums<G>(L, g, i, xi, sub, a, [&](int j, float (&t)[1]) {
+      const float4 xj = pv.s.x[j];
+      const float mj = pv.s.m[j], rhoj = pv.s.rho[j];
+      const int phj = pv.s.phase[j], fj = pv.s.flags[j];
+      settle(xj.x, xj.y, xj.z, mj, rhoj, phj, fj);
+      if (j == i || phj != target || (fj & kDying)) return;
+      const float r2 = norm2(pos_diff<KS>(xi, li, ld3(xj), pv.s.xlo, j));
+      if (r2 >= P.support2) return;
+      const float w = kW(P.kernel, sqrtf(r2));
+      t[0] = (mj / rhoj) * w;
+      const float wr = w / rhoj;
+      wr_max = wr > wr_max ? wr : wr_max;
+    });
+    for (int off = G / 2; off > 0; off >>= 1) {
+      const float o = __shfl_xor(wr_max, off, G);
+      wr_max = o > wr_max ? o : wr_max;
+    }
+    if (sub != 0) return;
+    const float wsum = a[0];
+    pv.t.w_norm[i] = wsum;
+    if (!(wsum > 0.0f)) {
+      pv.t.out_m[i] = 0.0f;
+    } else if (target == kVapor && P.pc_density_limit > 0.0f && !(fl & kDying) && wr_max > 0.0f) {
+      const float cap = P.pc_density_limit * wsum / wr_max;
+      if (pv.t.out_m[i] > cap) pv.t.out_m[i] = cap;
+    }
+  });
+}
+// Evaporated, condensed and merge partials of the normalised sources
+// (k_pc_normalize's sums).
+__global__ __launch_bounds__(kBlock) void k_pc_partials(PV pv, Count nc, double* partials, int stride) {
+  const int n = nc.get();
+  const int i = gtid();
+  double acc[3] = {0.0, 0.0, 0.0};
+  if (i < n) {
+    const uint8_t fl = pv.s.flags[i];
+    if (fl & kSource) {
+      const float om = pv.t.out_m[i];
+      if (!(fl & kDying)) {
+        if (fl & kTargetVapor) acc[0] = static_cast<double>(om);
+        else acc[1] = static_cast<double>(om);
+      }
+      if ((fl & kDying) && om > 0.0f) acc[2] = 1.0;
+    }
+  }
+  block_sums_store<3>(acc, partials, stride);
+}
+
 // Marks the cells holding a mass source (out_m > 0 after the normalisation)
 // by the phase its receivers have; the kind bits stay.
 __global__ __launch_bounds__(kBlock) void k_cell_sources(PV pv, GridDev g) {
@@ -255,6 +317,7 @@ __global__ __launch_bounds__(kBlock) void k_cell_sources(PV pv, GridDev g) {
 }
 
 // phase_change.cu:174-215
+// One thread per particle (many particles).
 template <bool KS>
 __global__ __launch_bounds__(kBlock) void k_pc_apply(PV pv, GridDev g, SimParams P, NbrList L, Count nc) {
   const int n = nc.get();
@@ -305,43 +368,103 @@ __global__ __launch_bounds__(kBlock) void k_pc_apply(PV pv, GridDev g, SimParams
   pv.s.m[i] = m_new;
 }
 
-// phase_change.cu:217-249 (pass 1)
-template <bool KS>
-__global__ __launch_bounds__(kBlock) void k_rebalance(PV pv, GridDev g, SimParams P, NbrList L, Count nc) {
-  const int n = nc.get();
-  const int i = gtid();
-  if (i >= n) return;
-  pv.t.out_m[i] = 0.0f;
-  pv.t.out_h[i] = 0.0f;
-  pv.t.ns[i] = st3(V3{0, 0, 0});
-  if (pv.s.phase[i] != kVapor) return;
-  const float beta = P.vapor_rebalance;
-  const V3 xi = ld3(pv.s.x[i]);
-  const V3 li = pos_lo<KS>(pv.s.xlo, i);
+// Fewer particles: a row of 16 lanes per receiver near a source giving mass to
+// its phase; one thread for the other fluid particles.
+__device__ inline void pc_apply_finish(const PV& pv, const SimParams& P, int i, float in_m, float in_H) {
+  const uint8_t ph = pv.s.phase[i];
   const float mi = pv.s.m[i];
-  const float hi = enthalpy(P, kVapor, pv.s.T[i]);
-  const V3 vi = ld3(pv.s.v[i]);
-  Acc<KS> dm, dH;
-  AccV3<KS> dP;
-  struct Nb {
-    float4 x, v;
-    float m, T;
-    int ph;
+  const float om_i = pv.t.out_m[i];
+  if ((pv.s.flags[i] & kDying) && om_i > 0.0f) {
+    pv.s.m[i] = 0.0f;
+    pv.s.phase[i] = kDead;
+    return;
+  }
+  if (!(om_i > 0.0f) && !(in_m > 0.0f)) return;
+  const float m_new = mi - om_i + in_m;
+  const float H_new = mi * enthalpy(P, ph, pv.s.T[i]) - om_i * pv.t.out_h[i] + in_H;
+  pv.s.T[i] = temp_from_h(P, ph, H_new / m_new);
+  pv.s.m[i] = m_new;
+}
+template <bool KS, int G>
+__global__ __launch_bounds__(kBlock) void k_pc_apply_lanes(PV pv, GridDev g, SimParams P, NbrList L, Count nc, int span) {
+  const int n = nc.get();
+  const int base = xcd_span(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x)) * span;
+  if (base >= n) return;  // uniform over the block
+  auto select = [&](int i) {
+    const uint8_t ph = pv.s.phase[i];
+    if (!is_fluid(ph)) return false;
+    if (!(pv.s.flags[i] & kDying) && cells_any(g, ld3(pv.s.x[i]), ph == kVapor ? kCellSrcV : kCellSrcL)) return true;
+    pc_apply_finish(pv, P, i, 0.0f, 0.0f);
+    return false;
   };
-  auto load = [&](int j) { return Nb{pv.s.x[j], pv.s.v[j], pv.s.m[j], pv.s.T[j], pv.s.phase[j]}; };
-  for_each_pair4(L, g, i, xi, load, [&](int j, const Nb d) {
-    if (j == i || d.ph != kVapor) return;
-    const float r2 = norm2(pos_diff<KS>(xi, li, ld3(d.x), pv.s.xlo, j));
-    if (r2 >= P.support2) return;
-    const float flow = beta * P.vol0 * kW(P.kernel, sqrtf(r2)) * (d.m - mi);
-    const bool from_j = flow > 0.0f;
-    dm += flow;
-    dH += flow * (from_j ? enthalpy(P, kVapor, d.T) : hi);
-    dP += (from_j ? ld3(d.v) : vi) * flow;
+  for_each_group<G>(base, span, n, select, [&](int i, int sub) {
+    const uint8_t ph = pv.s.phase[i];
+    const float Vi = pv.s.m[i] / pv.s.rho[i];
+    const V3 xi = ld3(pv.s.x[i]);
+    const V3 li = pos_lo<KS>(pv.s.xlo, i);
+    Acc<KS> a[2];
+    lane_sums<G>(L, g, i, xi, sub, a, [&](int j, float (&t)[2]) {
+      const float4 xj = pv.s.x[j];
+      const float om = pv.t.out_m[j], oh = pv.t.out_h[j], wn = pv.t.w_norm[j];
+      const int fj = pv.s.flags[j];
+      settle(xj.x, xj.y, xj.z, om, oh, wn, fj);
+      if (j == i) return;
+      if (!(om > 0.0f)) return;
+      const uint8_t target = (fj & kTargetVapor) ? kVapor : kLiquid;
+      if (target != ph) return;
+      const float r2 = norm2(pos_diff<KS>(xi, li, ld3(xj), pv.s.xlo, j));
+      if (r2 >= P.support2) return;
+      const float share = om * Vi * kW(P.kernel, sqrtf(r2)) / wn;
+      t[0] = share;
+      t[1] = share * oh;
+    });
+    if (sub == 0) pc_apply_finish(pv, P, i, float(a[0]), float(a[1]));
   });
-  pv.t.out_m[i] = float(dm);
-  pv.t.out_h[i] = float(dH);
-  pv.t.ns[i] = st3(V3(dP));
+}
+
+// phase_change.cu:217-249 (pass 1)
+// G lanes per vapour particle.
+template <bool KS, int G>
+__global__ __launch_bounds__(kBlock) void k_rebalance(PV pv, GridDev g, SimParams P, NbrList L, Count nc, int span) {
+  const int n = nc.get();
+  const int base = xcd_span(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x)) * span;
+  if (base >= n) return;  // uniform over the block
+  auto select = [&](int i) {
+    if (pv.s.phase[i] == kVapor) return true;
+    pv.t.out_m[i] = 0.0f;
+    pv.t.out_h[i] = 0.0f;
+    pv.t.ns[i] = st3(V3{0, 0, 0});
+    return false;
+  };
+  const float beta = P.vapor_rebalance;
+  for_each_group<G>(base, span, n, select, [&](int i, int sub) {
+    const V3 xi = ld3(pv.s.x[i]);
+    const V3 li = pos_lo<KS>(pv.s.xlo, i);
+    const float mi = pv.s.m[i];
+    const float hi = enthalpy(P, kVapor, pv.s.T[i]);
+    const V3 vi = ld3(pv.s.v[i]);
+    Acc<KS> a[5];  // mass, enthalpy, momentum
+    lane_sums<G>(L, g, i, xi, sub, a, [&](int j, float (&t)[5]) {
+      // every gather in flight together
+      const float4 x = pv.s.x[j], v = pv.s.v[j];
+      const float mj = pv.s.m[j], Tj = pv.s.T[j];
+      const int phj = pv.s.phase[j];
+      settle(x.x, x.y, x.z, v.x, v.y, v.z, mj, Tj, phj);
+      if (j == i || phj != kVapor) return;
+      const float r2 = norm2(pos_diff<KS>(xi, li, ld3(x), pv.s.xlo, j));
+      if (r2 >= P.support2) return;
+      const float flow = beta * P.vol0 * kW(P.kernel, sqrtf(r2)) * (mj - mi);
+      const bool from_j = flow > 0.0f;
+      const V3 dP = (from_j ? ld3(v) : vi) * flow;
+      t[0] = flow;
+      t[1] = flow * (from_j ? enthalpy(P, kVapor, Tj) : hi);
+      t[2] = dP.x, t[3] = dP.y, t[4] = dP.z;
+    });
+    if (sub != 0) return;
+    pv.t.out_m[i] = float(a[0]);
+    pv.t.out_h[i] = float(a[1]);
+    pv.t.ns[i] = st3(V3{float(a[2]), float(a[3]), float(a[4])});
+  });
 }
 
 // phase_change.cu:250-268 (pass 2) fused with mark_heavy_particles
@@ -715,20 +838,39 @@ void launch_kick_sources(const PV& pv, const SimParams& P, DevState* st, Count n
 int launch_pc_normalize(const PV& pv, const GridDev& g, const SimParams& P, const NbrList& L, Count n,
                         double* partials, int stride, hipStream_t s) {
   const int nb = blocks_for(n.ub > 0 ? n.ub : 1);
-  if (P.compensated) k_pc_normalize<true><<<nb, kBlock, 0, s>>>(pv, g, P, L, n, partials, stride);
-  else k_pc_normalize<false><<<nb, kBlock, 0, s>>>(pv, g, P, L, n, partials, stride);
+  if (rows_of_lanes(n.ub)) {
+    const int span = lane_span(n.ub), sb = (std::max(n.ub, 1) + span - 1) / span;
+    if (P.compensated) k_pc_normalize_lanes<true, 16><<<sb, kBlock, 0, s>>>(pv, g, P, L, n, span);
+    else k_pc_normalize_lanes<false, 16><<<sb, kBlock, 0, s>>>(pv, g, P, L, n, span);
+    k_pc_partials<<<nb, kBlock, 0, s>>>(pv, n, partials, stride);
+  } else {
+    if (P.compensated) k_pc_normalize<true><<<nb, kBlock, 0, s>>>(pv, g, P, L, n, partials, stride);
+    else k_pc_normalize<false><<<nb, kBlock, 0, s>>>(pv, g, P, L, n, partials, stride);
+  }
   return nb;
 }
 void launch_pc_apply(const PV& pv, const GridDev& g, const SimParams& P, const NbrList& L, Count n, hipStream_t s) {
   if (n.ub <= 0) return;
   if (g.num_cells > 0) k_cell_sources<<<blocks_for(g.num_cells), kBlock, 0, s>>>(pv, g);
-  if (P.compensated) k_pc_apply<true><<<blocks_for(n.ub), kBlock, 0, s>>>(pv, g, P, L, n);
-  else k_pc_apply<false><<<blocks_for(n.ub), kBlock, 0, s>>>(pv, g, P, L, n);
+  if (rows_of_lanes(n.ub)) {
+    const int span = lane_span(n.ub), nb = (n.ub + span - 1) / span;
+    if (P.compensated) k_pc_apply_lanes<true, 16><<<nb, kBlock, 0, s>>>(pv, g, P, L, n, span);
+    else k_pc_apply_lanes<false, 16><<<nb, kBlock, 0, s>>>(pv, g, P, L, n, span);
+  } else {
+    if (P.compensated) k_pc_apply<true><<<blocks_for(n.ub), kBlock, 0, s>>>(pv, g, P, L, n);
+    else k_pc_apply<false><<<blocks_for(n.ub), kBlock, 0, s>>>(pv, g, P, L, n);
+  }
 }
 void launch_rebalance(const PV& pv, const GridDev& g, const SimParams& P, const NbrList& L, Count n, hipStream_t s) {
   if (n.ub <= 0) return;
-  if (P.compensated) k_rebalance<true><<<blocks_for(n.ub), kBlock, 0, s>>>(pv, g, P, L, n);
-  else k_rebalance<false><<<blocks_for(n.ub), kBlock, 0, s>>>(pv, g, P, L, n);
+  const int span = lane_span(n.ub), nb = (n.ub + span - 1) / span;
+  if (rows_of_lanes(n.ub)) {
+    if (P.compensated) k_rebalance<true, 16><<<nb, kBlock, 0, s>>>(pv, g, P, L, n, span);
+    else k_rebalance<false, 16><<<nb, kBlock, 0, s>>>(pv, g, P, L, n, span);
+  } else {
+    if (P.compensated) k_rebalance<true, 4><<<nb, kBlock, 0, s>>>(pv, g, P, L, n, span);
+    else k_rebalance<false, 4><<<nb, kBlock, 0, s>>>(pv, g, P, L, n, span);
+  }
 }
 void launch_rebalance_apply_mark(const PV& pv, const SimParams& P, Count n, bool rebalance, uint32_t* flag,
                                  hipStream_t s) {

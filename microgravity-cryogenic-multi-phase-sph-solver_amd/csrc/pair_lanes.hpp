@@ -35,13 +35,13 @@ __device__ inline float powf_cr(float x, float y) { return static_cast<float>(po
 // operand).  The sums therefore see the reference's order, whatever G is.
 template <int G>
 struct Lanes {
-  static_assert(G == 1 || G == 2 || G == 4, "groups of one quad at most");
+  static_assert(G == 1 || G == 2 || G == 4 || G == 16, "a quad's parts, or a row of 16 lanes");
   // every lane of the group gets lane k's v
   template <int K>
   __device__ static inline float from(float v) {
     if constexpr (G == 1) return v;
-    constexpr int a = G == 4 ? K : K, b = G == 4 ? K : 2 + K;
-    constexpr int ctrl = a | (a << 2) | (b << 4) | (b << 6);
+    constexpr int b = G == 2 ? 2 + K : K;
+    constexpr int ctrl = G == 16 ? 0x150 + K : K | (K << 2) | (b << 4) | (b << 6);  // row_newbcast or quad_perm
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, 0xf, 0xf, true));
   }
   template <int K>
@@ -95,6 +95,73 @@ __device__ inline int xcd_span(int b, int nblocks) {
   if (b >= nblocks / span * span) return b;
   return b / span * span + (b % 8) * kSpanChunk + (b / 8) % kSpanChunk;
 }
+
+// Orders this wave's LDS writes before its later reads (the hardware does; this
+// keeps the compiler from moving them).
+__device__ inline void wave_lds_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
+
+// One block's particles [base, base + span), span <= kBlock: select(i) says
+// whether particle i takes part (and writes what the others get); the selected
+// ones, in order, go to groups of G lanes, body(i, sub) once per lane of a
+// group.  Every thread of the block calls it.
+template <int G, class Select, class Body>
+__device__ inline void for_each_group(int base, int span, int n, Select&& select, Body&& body) {
+  __shared__ int s_work[kBlock], s_tot[kBlock / 64];
+  const int t = static_cast<int>(threadIdx.x), lane = t & 63, wave = t >> 6;
+  const bool keep = t < span && base + t < n && select(base + t);
+  const unsigned long long kept = __ballot(keep);
+  if (lane == 0) s_tot[wave] = __popcll(kept);
+  __syncthreads();
+  int first = 0, total = 0;
+  for (int w = 0; w < kBlock / 64; ++w) {
+    const int c = s_tot[w];
+    first += w < wave ? c : 0;
+    total += c;
+  }
+  if (keep) s_work[first + __popcll(kept & ((1ull << lane) - 1ull))] = base + t;
+  __syncthreads();
+  for (int slot = t / G; slot < total; slot += kBlock / G) body(s_work[slot], t % G);
+}
+
+// Sums over particle i's neighbours by its group of G lanes: eval(j, t) sets
+// the terms t[0..N) of neighbour j (they come in as zeros), which are added to
+// acc in list order.  Without a complete list every lane walks the 27 cells.
+template <int G, int N, bool KS, class Eval>
+__device__ inline void lane_sums(const NbrList& L, const GridDev& g, int i, V3 xi, int sub, Acc<KS> (&acc)[N],
+                                 Eval&& eval) {
+  const int c = L.valid ? L.count[i] : -1;
+  if (c < 0) {
+    for_each_nbr(g, xi, [&](int j) {
+      float t[N] = {};
+      eval(j, t);
+#pragma unroll
+      for (int q = 0; q < N; ++q) acc[q] += t[q];
+    });
+    return;
+  }
+  const int* lp = reinterpret_cast<const int*>(list_chunks(L, i));
+  int jn = sub < c ? lp[(sub >> 2) * (4 * kListGroup) + (sub & 3)] : -1;
+  for (int e = sub; e - sub < c; e += G) {
+    const int j = take(jn);
+    jn = e + G < c ? lp[((e + G) >> 2) * (4 * kListGroup) + ((e + G) & 3)] : -1;
+    float t[N] = {};
+    if (j >= 0) eval(j, t);
+    unrolled<G>([&](auto kc) {
+#pragma unroll
+      for (int q = 0; q < N; ++q) acc[q] += Lanes<G>::template from<decltype(kc)::value>(t[q]);
+    });
+  }
+}
+// The phase-change and rebalance passes take a row of 16 lanes per particle
+// while the chip is not full (their time is one particle's chain of dependent
+// gathers then), with particles per block so that a group has one to four of
+// them.  26 k particles: normalise 42 -> 7 us (and 5 for its partials), apply
+// 43 -> 11, rebalance 40 -> 10; 188 k: 47 -> 21, 43 -> 23, 56 -> 51.  Beyond,
+// normalise and apply are faster with one thread per particle (1.2 M: 63
+// against 132 us, 117 against 125), rebalance with a quad (245 against 278).
+constexpr int kLanesWide = 250000;
+inline bool rows_of_lanes(int n) { return n < kLanesWide; }
+inline int lane_span(int n) { return n < 60000 ? 16 : n < kLanesWide ? 64 : kBlock; }
 
 }  // namespace
 }  // namespace cryo
