@@ -41,7 +41,7 @@ struct FluidConst {
 // grid
 void launch_kick_drift_keys(const PV& pv, const GridDev& g, DevState* st, Count n, bool do_kick, bool continuity,
                             bool tvf, uint32_t* keys, uint32_t* vals, hipStream_t s);
-int radix_tiles(int n);
+int radix_tiles(int n);  // the most tiles a sort of up to n keys takes
 void launch_radix_sort(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32_t* vals_alt, Count n,
                        int key_bits, uint32_t* tile_hist, uint32_t* row_total, hipStream_t s, bool* result_in_alt);
 void launch_cell_offsets(const uint32_t* keys, Count n, int num_cells, int* off, DevState* st, hipStream_t s);

@@ -5,6 +5,8 @@
 // (spatial_hash.cu:48-171).  The reference CPU path sorts with a serial stable
 // counting sort; any stable sort by the same key gives the same permutation,
 // so this LSD radix sort (8-bit digits, stable per pass) is bit-exact with it.
+#include <algorithm>
+
 #include "kernels.hpp"
 
 namespace cryo {
@@ -51,10 +53,14 @@ __global__ __launch_bounds__(kBlock) void k_kick_drift_keys(PV pv, GridDev g, De
 }
 
 // ------------------------------------------------------------- radix sort
+// A tile's keys are ranked round by round (three barriers each), so few keys
+// take short tiles, which also spread over more CUs: a scatter of 26 k keys
+// takes 20 us with 16 rounds and 8 with 4.
 constexpr int kRsThreads = 256;
-constexpr int kRsItems = 16;
-constexpr int kRsTile = kRsThreads * kRsItems;
+constexpr int kRsItems = 16, kRsItemsFew = 4;
+constexpr int kRsFew = 400000;  // keys from which the long tiles are used
 
+template <int ITEMS>
 __global__ __launch_bounds__(kRsThreads) void k_radix_hist(const uint32_t* keys, Count nc, int shift,
                                                           uint32_t* tile_hist, int num_tiles) {
   const int n = nc.get();
@@ -62,8 +68,8 @@ __global__ __launch_bounds__(kRsThreads) void k_radix_hist(const uint32_t* keys,
   const int tid = threadIdx.x;
   h[tid] = 0;
   __syncthreads();
-  const int base = blockIdx.x * kRsTile;
-  for (int k = 0; k < kRsItems; ++k) {
+  const int base = blockIdx.x * kRsThreads * ITEMS;
+  for (int k = 0; k < ITEMS; ++k) {
     const int i = base + k * kRsThreads + tid;
     if (i < n) atomicAdd(&h[(keys[i] >> shift) & 255u], 1u);
   }
@@ -128,6 +134,7 @@ __global__ __launch_bounds__(256) void k_radix_scan_rows(uint32_t* tile_hist, in
 
 // Stable scatter: ranks inside a tile follow element order (round by round,
 // wave by wave, lane by lane), tiles follow tile order through tile_off.
+template <int ITEMS>
 __global__ __launch_bounds__(kRsThreads) void k_radix_scatter(const uint32_t* keys_in, const uint32_t* vals_in,
                                                              uint32_t* keys_out, uint32_t* vals_out, Count nc,
                                                              int shift, const uint32_t* tile_off, int num_tiles,
@@ -154,9 +161,9 @@ __global__ __launch_bounds__(kRsThreads) void k_radix_scatter(const uint32_t* ke
   running[tid] = 0;
   for (int w = 0; w < kRsThreads / 64; ++w) wave_cnt[w][tid] = 0;
   __syncthreads();
-  const int base = blockIdx.x * kRsTile;
+  const int base = blockIdx.x * kRsThreads * ITEMS;
   const uint64_t lt_mask = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
-  for (int k = 0; k < kRsItems; ++k) {
+  for (int k = 0; k < ITEMS; ++k) {
     const int i = base + k * kRsThreads + tid;
     const bool valid = i < n;
     const uint32_t key = valid ? keys_in[i] : 0u;
@@ -275,18 +282,27 @@ void launch_kick_drift_keys(const PV& pv, const GridDev& g, DevState* st, Count 
                                                      tvf ? 1 : 0, keys, vals);
 }
 
-int radix_tiles(int n) { return (n + kRsTile - 1) / kRsTile; }
+static int rs_tiles(int n) {
+  const int tile = kRsThreads * (n < kRsFew ? kRsItemsFew : kRsItems);
+  return (n + tile - 1) / tile;
+}
+int radix_tiles(int n) { return std::max(rs_tiles(n), rs_tiles(std::min(n, kRsFew - 1))); }
 
 void launch_radix_sort(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32_t* vals_alt, Count n,
                        int key_bits, uint32_t* tile_hist, uint32_t* row_total, hipStream_t s, bool* result_in_alt) {
   *result_in_alt = false;
   if (n.ub <= 0) return;
-  const int tiles = radix_tiles(n.ub);
+  const int tiles = rs_tiles(n.ub);
+  const bool few = n.ub < kRsFew;
   uint32_t *ki = keys, *vi = vals, *ko = keys_alt, *vo = vals_alt;
   for (int shift = 0; shift < key_bits; shift += 8) {
-    k_radix_hist<<<tiles, kRsThreads, 0, s>>>(ki, n, shift, tile_hist, tiles);
+    if (few) k_radix_hist<kRsItemsFew><<<tiles, kRsThreads, 0, s>>>(ki, n, shift, tile_hist, tiles);
+    else k_radix_hist<kRsItems><<<tiles, kRsThreads, 0, s>>>(ki, n, shift, tile_hist, tiles);
     k_radix_scan_rows<<<256, 256, 0, s>>>(tile_hist, tiles, row_total);
-    k_radix_scatter<<<tiles, kRsThreads, 0, s>>>(ki, vi, ko, vo, n, shift, tile_hist, tiles, row_total);
+    if (few)
+      k_radix_scatter<kRsItemsFew><<<tiles, kRsThreads, 0, s>>>(ki, vi, ko, vo, n, shift, tile_hist, tiles, row_total);
+    else
+      k_radix_scatter<kRsItems><<<tiles, kRsThreads, 0, s>>>(ki, vi, ko, vo, n, shift, tile_hist, tiles, row_total);
     uint32_t* t = ki;
     ki = ko;
     ko = t;
