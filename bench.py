@@ -499,8 +499,8 @@ def main():
     # instruction over the SIMD-cycles of the live launch time.  Counter-based
     # fields are given only for the workload the profiles were taken on.
     on_profile = abs(a.dx - C2_DX) < 1e-9
-    traffic = profile_column("hbm_traffic_c2.txt", "k_forces_tiled", 1) if on_profile else None
-    valu_instr = profile_column("valu_l2_c2.txt", "k_forces_tiled", 2) if on_profile else None
+    traffic = profile_column("hbm_traffic_c2.txt", "k_forces<", 1) if on_profile else None
+    valu_instr = profile_column("valu_l2_c2.txt", "k_forces<", 2) if on_profile else None
     valu_frac = (valu_instr * 4 / SIMDS / (forces_ms * 1e-3 * VALU_CLOCK_HZ)) if valu_instr else None
     tfrac = (traffic / (forces_ms * 1e-3) / 1e9 / HBM_PEAK_GBS) if traffic else None
     if valu_frac is None:
@@ -519,8 +519,8 @@ def main():
                 "valu_source": "profiles/valu_l2_c2.txt (SQ_INSTS_VALU per launch) over the live kernel time"
                 if valu_frac is not None else None,
                 "limiter": limiter,
-                "kernel": "k_forces_tiled (transport velocity + momentum + wall loads + continuity + dt "
-                          "maxima; LDS-staged cell tiles) + its overflow instance",
+                "kernel": "k_forces (transport velocity + momentum + wall loads + continuity + dt "
+                          "maxima; lanes of a wave share a particle) + its overflow sweep",
                 "kernel_ms": forces_ms, "algorithmic_bytes": forces_bytes}
     out = {
         "metric": "particle-steps/s + % HBM roofline at 1M; ensemble speedup; adjoint/forward cost",

@@ -722,8 +722,8 @@ PYBIND11_MODULE(CryoSPH, m) {
         check(r);
         return py::make_tuple(v, py::make_tuple(ms[0], ms[1], ms[2], ms[3]));
       }, py::arg("trial_steps") = 5,
-         "Times trial_steps steps of each launch variant of the neighbour passes (LDS cell tiles or list "
-         "gathers, for forces and interface), keeps the fastest, restores the state; returns (variant, "
+         "Times trial_steps steps of each launch variant of the neighbour passes (lanes per particle of "
+         "the forces pass; LDS cell tiles or list gathers for the interface pass), keeps the fastest, restores the state; returns (variant, "
          "ms per step of variants 0..3).  Results do not depend on the variant.")
       .def_property("launch_variant", [](Solver& S) {
         int32_t v = 0;
