@@ -58,7 +58,10 @@ __global__ __launch_bounds__(kBlock) void k_kick_drift_keys(PV pv, GridDev g, De
 // takes 20 us with 16 rounds and 8 with 4.
 constexpr int kRsThreads = 256;
 constexpr int kRsItems = 16, kRsItemsFew = 4;
-constexpr int kRsFew = 400000;  // keys from which the long tiles are used
+// Keys from which the long tiles are used.  A scatter of 1.2 M keys took 24 us
+// with them and 12 with short ones too, so the line can go once the sort has
+// been compared at full size with short tiles alone.
+constexpr int kRsFew = 400000;
 
 template <int ITEMS>
 __global__ __launch_bounds__(kRsThreads) void k_radix_hist(const uint32_t* keys, Count nc, int shift,
