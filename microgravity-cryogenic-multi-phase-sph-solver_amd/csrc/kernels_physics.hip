@@ -541,13 +541,18 @@ __device__ inline float interface_particle(const PV& pv, const SimParams& P, int
 // neighbours are summed.  Bitwise the full pass's results (adding a zero to a
 // running sum that starts at +0 never changes it).  Resets the dt maxima.
 // A row of 16 lanes per particle that has a wall or the other phase nearby, up
-// to kInterfaceLanes particles: 26 k 66 -> 26 us, 4 k 77 -> 15; 188 k would
-// take 102 us with it, 88 with one thread per particle (13 ordered sums, each
-// repeated by 16 lanes).
-constexpr int kInterfaceLanes = 100000;
+// to kInterfaceLanes particles (kInterfaceLanesKs in the precision form, whose
+// compensated additions cost four times a plain one and are repeated by all 16
+// lanes): 13 ordered sums.  A block takes one particle per row: spans of 64, and
+// with them four particles in turn for some rows, took 78 us at 70 k.
+// us with the row / with one thread per particle, two-phase spheres:
+//   plain  6 k 16 / 78, 26 k 27 / 66, 60 k 46 / 72, 100 k 69 / 81, 140 k 86 / 87, 188 k 106 / 87
+//   precise  6 k 40 / 130, 20 k 71 / 101, 26 k 100 / 101, 45 k 120 / 105, 100 k 224 / 120
+constexpr int kInterfaceLanes = 140000, kInterfaceLanesKs = 25000;
 template <bool KS, int G>
 __global__ __launch_bounds__(kBlock) void k_interface_lanes(PV pv, GridDev g, SimParams P, NbrList L, DevState* st,
-                                                            Count nc, int csf_mode, int span) {
+                                                            Count nc, int csf_mode) {
+  constexpr int span = kBlock / G;
   const int n = nc.get();
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     for (int k = 0; k < 5; ++k) st->max_bits[k] = 0u;
@@ -1134,10 +1139,10 @@ int launch_interface(const PV& pv, const GridDev& g, const SimParams& P, const N
   const int nb = blocks_for(n.ub > 0 ? n.ub : 1);
   const int cm = csf_mode ? 1 : 0;
   if (P.st_model != 2 && !P.sps && L.valid && g.flags) {
-    if (n.ub < kInterfaceLanes) {
-      const int span = lane_span(n.ub), sb = (std::max(n.ub, 1) + span - 1) / span;
-      if (P.compensated) k_interface_lanes<true, 16><<<sb, kBlock, 0, s>>>(pv, g, P, L, st, n, cm, span);
-      else k_interface_lanes<false, 16><<<sb, kBlock, 0, s>>>(pv, g, P, L, st, n, cm, span);
+    if (n.ub < (P.compensated ? kInterfaceLanesKs : kInterfaceLanes)) {
+      const int sb = blocks_for(16ll * std::max(n.ub, 1));
+      if (P.compensated) k_interface_lanes<true, 16><<<sb, kBlock, 0, s>>>(pv, g, P, L, st, n, cm);
+      else k_interface_lanes<false, 16><<<sb, kBlock, 0, s>>>(pv, g, P, L, st, n, cm);
       if (heat_partials) k_heat_partials<<<nb, kBlock, 0, s>>>(pv, n, heat_partials);
     } else {
       if (P.compensated) k_interface_sparse<true><<<nb, kBlock, 0, s>>>(pv, g, P, L, st, n, cm, heat_partials);

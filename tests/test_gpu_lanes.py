@@ -1,5 +1,6 @@
 """The neighbour passes with several lanes per particle, bit for bit against the
-FP32 oracle where they can go wrong: both group sizes; particle counts that leave
+FP32 oracle (the precision form, which has none, against its other forms) where
+they can go wrong: both group sizes; particle counts that leave
 partial groups, waves and blocks; lists that overflow (the cell sweep); pairs
 outside the fast arithmetic's range (coincident and nearly coincident
 particles, an infinite temperature, fluid at rest), whose targets are done
@@ -130,3 +131,61 @@ def test_both_sides_of_the_size_rules(n):
     for f in FIELDS + ("m", "alpha", "wall_w", "heat_w", "nrm", "ns", "id"):
         a, b = gpu.field(f), cpu.field(f)
         assert np.array_equal(a, b, equal_nan=True), (f, int((a != b).sum()))
+
+
+def beside(ps, dx, n):
+    """ps and a block of isolated walls (1.2 dx apart, none within reach of the tank) that makes n particles of it."""
+    pad = n - len(ps)
+    assert pad >= 0
+    side = int(np.ceil(max(pad, 1) ** (1 / 3)))
+    g = np.stack(np.meshgrid(*[np.arange(side)] * 3, indexing="ij"), -1).reshape(-1, 3)[:pad]
+    x = ps.x.max(0) + np.float32(6 * dx) + (1.2 * dx * g).astype(np.float32)
+    cat = lambda a, b: np.concatenate([a, np.asarray(b, a.dtype)])  # noqa: E731
+    z = np.zeros(pad)
+    return cabi.ParticleSet(cat(ps.x, x), cat(ps.v, 0 * x), cat(ps.nrm, 0 * x), cat(ps.m, z + ps.m.max()),
+                            cat(ps.rho, z + ps.rho.max()), cat(ps.T, z + ps.T[0]), cat(ps.phase, z + cabi.WALL),
+                            cat(ps.flags, z), None)
+
+
+@pytest.mark.parametrize("n", [30_000, 65_000, 80_000, 160_000, 310_000, 610_000])
+@pytest.mark.parametrize("compensated", [0, 1])
+@pytest.mark.parametrize("crowd", [False, True])
+def test_the_form_a_size_selects_changes_no_bit(crowd, compensated, n):
+    """A superheated two-phase tank of 13 k particles, alone and beside enough
+    walls, out of its reach, that every pass takes the form it has for n
+    particles: the tank's fields are the same bits, in the precision form too
+    (which has no FP32 oracle), and where lists overflow."""
+    fluid = cabi.hip_fluid_preset("LN2")
+    dx = 0.004
+    cfg = cabi.default_config(dx=dx, gravity=(0, 0, -0.5), contact_angle_deg=20, velocity_scale=1.0, thermo_mode=0,
+                              lee_evaporation=5.0, lee_condensation=5.0, compensated_sums=compensated)
+    ps = cabi.hip_build_tank_particles(cabi.box(0.07, 0.07, 0.07), fluid, dx, cabi.default_fill(T_liquid=fluid.T_sat + 2.0))
+    rng = np.random.default_rng(5)
+    fl = ps.phase != cabi.WALL
+    ps.x[fl] += (0.05 * dx * rng.uniform(-1, 1, (int(fl.sum()), 3))).astype(np.float32)
+    ps.v[fl] = rng.normal(0, 0.05, (int(fl.sum()), 3)).astype(np.float32)
+    if crowd:  # more than 96 neighbours each, liquid and vapour, at the interface
+        for ph, side in ((cabi.LIQUID, -1), (cabi.VAPOR, 1)):
+            at = np.flatnonzero(ps.phase == ph)
+            at = at[np.argsort(side * ps.x[at, 2], kind="stable")[:120]]
+            ps.x[at] = ps.x[at].mean(0) + (0.5 * dx * rng.uniform(-1, 1, (120, 3))).astype(np.float32)
+    print("lanes form", crowd, compensated, n, len(ps), flush=True)
+    big = beside(ps, dx, n)
+    lo, hi = big.x.min(0) - 4 * dx, big.x.max(0) + 4 * dx
+    edge = ps.x.max() + 3 * dx
+
+    def fields(p, variant):
+        s = cabi.HipSolver(cfg, fluid)
+        s.set_launch_variant(variant)
+        s.set_particles(p, lo, hi)
+        s.run_steps(1 if crowd else 3)
+        assert s.diagnostics().evaporated_mass > 0
+        tank = s.field("x").max(1) < edge
+        return {f: s.field(f)[tank] for f in FIELDS + ("m", "alpha", "wall_w", "out_m", "out_h", "w_norm", "nrm", "ns", "rmin")}
+
+    alone = fields(ps, 0)
+    assert np.isfinite(alone["x"]).all()
+    for variant in (0, 1):
+        got = fields(big, variant)
+        for f, a in alone.items():
+            assert np.array_equal(a, got[f], equal_nan=True), (f, variant, int((a != got[f]).sum()))
