@@ -423,9 +423,19 @@ __global__ __launch_bounds__(kBlock) void k_pc_apply_lanes(PV pv, GridDev g, Sim
 }
 
 // phase_change.cu:217-249 (pass 1)
-// G lanes per vapour particle.
+// G lanes per vapour particle, one particle per group of a block: a row of 16
+// while its shorter chain counts, a quad beyond (all G lanes repeat the five
+// ordered sums, four times as dear where they are compensated).
+// us with the row / the quad / one thread per particle, two-phase spheres:
+//   plain  13 k 8 / 16 / 38, 45 k 16 / 17 / 43, 62 k 17 / 19 / 44, 120 k 26 / 27 / 45,
+//          293 k 54 / 48 / 73, 1.2 M - / 216 / 284
+//   precise  13 k 18 / 25 / 53, 26 k 18..37 / 26 / 54, 62 k 51 / 32 / 58, 188 k 122 / 55 / 79,
+//          293 k 182 / 77 / 100, 1.2 M - / 298 / 416
+// (Quads with 256 particles a block, four in turn each: 293 k 63 and 121 us.)
+constexpr int kRebalanceRow = 60000, kRebalanceRowKs = 20000;
 template <bool KS, int G>
-__global__ __launch_bounds__(kBlock) void k_rebalance(PV pv, GridDev g, SimParams P, NbrList L, Count nc, int span) {
+__global__ __launch_bounds__(kBlock) void k_rebalance(PV pv, GridDev g, SimParams P, NbrList L, Count nc) {
+  constexpr int span = kBlock / G;
   const int n = nc.get();
   const int base = xcd_span(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x)) * span;
   if (base >= n) return;  // uniform over the block
@@ -863,13 +873,14 @@ void launch_pc_apply(const PV& pv, const GridDev& g, const SimParams& P, const N
 }
 void launch_rebalance(const PV& pv, const GridDev& g, const SimParams& P, const NbrList& L, Count n, hipStream_t s) {
   if (n.ub <= 0) return;
-  const int span = lane_span(n.ub), nb = (n.ub + span - 1) / span;
-  if (rows_of_lanes(n.ub)) {
-    if (P.compensated) k_rebalance<true, 16><<<nb, kBlock, 0, s>>>(pv, g, P, L, n, span);
-    else k_rebalance<false, 16><<<nb, kBlock, 0, s>>>(pv, g, P, L, n, span);
+  const bool row = n.ub < (P.compensated ? kRebalanceRowKs : kRebalanceRow);
+  const int nb = blocks_for((row ? 16ll : 4ll) * n.ub);
+  if (P.compensated) {
+    if (row) k_rebalance<true, 16><<<nb, kBlock, 0, s>>>(pv, g, P, L, n);
+    else k_rebalance<true, 4><<<nb, kBlock, 0, s>>>(pv, g, P, L, n);
   } else {
-    if (P.compensated) k_rebalance<true, 4><<<nb, kBlock, 0, s>>>(pv, g, P, L, n, span);
-    else k_rebalance<false, 4><<<nb, kBlock, 0, s>>>(pv, g, P, L, n, span);
+    if (row) k_rebalance<false, 16><<<nb, kBlock, 0, s>>>(pv, g, P, L, n);
+    else k_rebalance<false, 4><<<nb, kBlock, 0, s>>>(pv, g, P, L, n);
   }
 }
 void launch_rebalance_apply_mark(const PV& pv, const SimParams& P, Count n, bool rebalance, uint32_t* flag,
