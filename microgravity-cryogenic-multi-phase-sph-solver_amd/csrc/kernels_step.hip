@@ -241,11 +241,15 @@ __global__ __launch_bounds__(kBlock) void k_pc_normalize(PV pv, GridDev g, SimPa
   block_sums_store<3>(acc, partials, stride);
 }
 
-// The same for fewer particles: a row of 16 lanes per source, then the partials
-// (k_pc_partials).
+// The same for fewer particles: a row of 16 lanes per source, 16 particles a
+// block (few of them are sources), then the partials (k_pc_partials, 5 us up to
+// 600 k, 10 at 1.2 M).  us without them / with one thread per particle, two-phase
+// spheres: plain 26 k 7 / 40, 188 k 11 / 46, 293 k 14 / 46, 600 k 25 / 38,
+// 1.2 M 43 / 50; precise 26 k 9 / 51, 188 k 17 / 58, 600 k 32 / 49, 1.2 M 49 / 57.
+constexpr int kNormalizeLanes = 600000;
 template <bool KS, int G>
-__global__ __launch_bounds__(kBlock) void k_pc_normalize_lanes(PV pv, GridDev g, SimParams P, NbrList L, Count nc,
-                                                              int span) {
+__global__ __launch_bounds__(kBlock) void k_pc_normalize_lanes(PV pv, GridDev g, SimParams P, NbrList L, Count nc) {
+  constexpr int span = kBlock / G;
   const int n = nc.get();
   const int base = xcd_span(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x)) * span;
   if (base >= n) return;  // uniform over the block
@@ -369,7 +373,13 @@ __global__ __launch_bounds__(kBlock) void k_pc_apply(PV pv, GridDev g, SimParams
 }
 
 // Fewer particles: a row of 16 lanes per receiver near a source giving mass to
-// its phase; one thread for the other fluid particles.
+// its phase; one thread for the other fluid particles.  16 particles a block, from
+// kApplyWide on 32 (fewer blocks that find nothing to do; in the precision form,
+// where a receiver costs more, 16 stay the better).  us with 16 / with 32 / with
+// one thread per particle, two-phase spheres:
+//   plain  26 k 13 / 15 / 42, 62 k 16 / 14 / 35, 188 k 36 / 26 / 44, 293 k 56 / 38 / 47, 450 k 80 / 49 / 40
+//   precise  26 k 16 / 23 / 50, 120 k 33 / 44 / 52, 150 k 36 / 44 / 39, 188 k 47 / 49 / 53, 240 k 59 / 52 / 46
+constexpr int kApplyLanes = 300000, kApplyLanesKs = 150000, kApplyWide = 60000;
 __device__ inline void pc_apply_finish(const PV& pv, const SimParams& P, int i, float in_m, float in_H) {
   const uint8_t ph = pv.s.phase[i];
   const float mi = pv.s.m[i];
@@ -848,10 +858,10 @@ void launch_kick_sources(const PV& pv, const SimParams& P, DevState* st, Count n
 int launch_pc_normalize(const PV& pv, const GridDev& g, const SimParams& P, const NbrList& L, Count n,
                         double* partials, int stride, hipStream_t s) {
   const int nb = blocks_for(n.ub > 0 ? n.ub : 1);
-  if (rows_of_lanes(n.ub)) {
-    const int span = lane_span(n.ub), sb = (std::max(n.ub, 1) + span - 1) / span;
-    if (P.compensated) k_pc_normalize_lanes<true, 16><<<sb, kBlock, 0, s>>>(pv, g, P, L, n, span);
-    else k_pc_normalize_lanes<false, 16><<<sb, kBlock, 0, s>>>(pv, g, P, L, n, span);
+  if (n.ub < kNormalizeLanes) {
+    const int lb = blocks_for(16ll * std::max(n.ub, 1));
+    if (P.compensated) k_pc_normalize_lanes<true, 16><<<lb, kBlock, 0, s>>>(pv, g, P, L, n);
+    else k_pc_normalize_lanes<false, 16><<<lb, kBlock, 0, s>>>(pv, g, P, L, n);
     k_pc_partials<<<nb, kBlock, 0, s>>>(pv, n, partials, stride);
   } else {
     if (P.compensated) k_pc_normalize<true><<<nb, kBlock, 0, s>>>(pv, g, P, L, n, partials, stride);
@@ -862,8 +872,8 @@ int launch_pc_normalize(const PV& pv, const GridDev& g, const SimParams& P, cons
 void launch_pc_apply(const PV& pv, const GridDev& g, const SimParams& P, const NbrList& L, Count n, hipStream_t s) {
   if (n.ub <= 0) return;
   if (g.num_cells > 0) k_cell_sources<<<blocks_for(g.num_cells), kBlock, 0, s>>>(pv, g);
-  if (rows_of_lanes(n.ub)) {
-    const int span = lane_span(n.ub), nb = (n.ub + span - 1) / span;
+  if (n.ub < (P.compensated ? kApplyLanesKs : kApplyLanes)) {
+    const int span = P.compensated || n.ub < kApplyWide ? 16 : 32, nb = (n.ub + span - 1) / span;
     if (P.compensated) k_pc_apply_lanes<true, 16><<<nb, kBlock, 0, s>>>(pv, g, P, L, n, span);
     else k_pc_apply_lanes<false, 16><<<nb, kBlock, 0, s>>>(pv, g, P, L, n, span);
   } else {

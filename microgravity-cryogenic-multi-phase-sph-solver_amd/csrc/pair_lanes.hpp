@@ -152,15 +152,6 @@ __device__ inline void lane_sums(const NbrList& L, const GridDev& g, int i, V3 x
     });
   }
 }
-// The phase-change passes take a row of 16 lanes per particle while the chip is
-// not full (their time is one particle's chain of dependent gathers then), with
-// particles per block so that a group has one to four of them.  26 k particles:
-// normalise 42 -> 7 us (and 5 for its partials), apply 43 -> 11; 188 k: 47 -> 21,
-// 43 -> 23.  Beyond, normalise and apply are faster with one thread per particle
-// (1.2 M: 63 against 132 us, 117 against 125).
-constexpr int kLanesWide = 250000;
-inline bool rows_of_lanes(int n) { return n < kLanesWide; }
-inline int lane_span(int n) { return n < 60000 ? 16 : n < kLanesWide ? 64 : kBlock; }
 
 }  // namespace
 }  // namespace cryo
