@@ -1172,13 +1172,21 @@ void launch_heat_norm(DevState* st, const double* partials, int nb, bool active,
 
 // Lanes per particle of the forces pass: four while the chip is not full
 // (shorter chains), two beyond (each lane of a group repeats the ordered
-// additions).  26 k particles 0.59 against 0.62 ms a step, 188 k particles
-// 0.89 against 0.87, 1.2 M 3.5 against 3.1.  `other` takes the other count.
-int forces_lanes(int n, bool other) { return (n < 120000) != other ? 4 : 2; }
+// additions, four times as dear in the precision form).  us with four / two:
+//   CSF  45 k 56 / 72, 60 k 65 / 76, 80 k 85 / 81, 110 k 101 / 100, 188 k 149 / 145, 600 k 403 / 356
+//   CSF, precise  26 k 67 / 88, 40 k 85 / 88, 60 k 113 / 91, 120 k 180 / 151, 600 k 682 / 513
+//   no tension  60 k 48 / 57, 120 k 72 / 77, 233 k 107 / 110, 297 k 139 / 128
+//   no tension, SPS  61 k 52 / 68, 150 k 94 / 91, 233 k 139 / 144, 297 k 183 / 160
+//   Akinci  34 k 70 / 92, 113 k 161 / 183, 217 k 265 / 270, 299 k 364 / 354, 489 k 565 / 526
+// `other` takes the other count.
+int forces_lanes(const SimParams& P, bool csf_mode, int n, bool other) {
+  const int below = P.compensated ? 50000 : csf_mode ? 75000 : 250000;
+  return (n < below) != other ? 4 : 2;
+}
 
 void launch_forces(const PV& pv, const GridDev& g, const SimParams& P, const NbrList& L, DevState* st, Count n,
                    bool csf_mode, bool akinci, bool continuity, bool thermal, bool other_lanes, hipStream_t s) {
-  const int lanes = forces_lanes(n.ub, other_lanes);
+  const int lanes = forces_lanes(P, csf_mode, n.ub, other_lanes);
   if (akinci) launch_forces_akinci(pv, g, P, L, st, n, continuity, thermal, lanes, s);
   else if (csf_mode) launch_forces_csf(pv, g, P, L, st, n, continuity, thermal, lanes, s);
   else launch_forces_none(pv, g, P, L, st, n, continuity, thermal, lanes, s);
