@@ -250,8 +250,11 @@ __global__ __launch_bounds__(kBlock) void k_density(PV pv, GridDev g, SimParams 
 
 // One thread per particle: what very large sets take (from kDensWide on, where
 // every SIMD is full either way and the shorter chains of the row of lanes
-// above no longer pay for its bookkeeping: 2.2 M particles 1120 us with it).
-constexpr int kDensWide = 700000;
+// above no longer pay for its bookkeeping).  us with the row / with one thread:
+//   two-phase sphere  188 k 131 / 184, 420 k 273 / 287, 550 k 361 / 373, 700 k 455 / 444, 1.2 M 787 / 693
+//   precise  188 k 183 / 256, 420 k 387 / 467, 550 k 501 / 548, 700 k 633 / 628, 1.2 M 1099 / 1019
+//   column  297 k 131 / 176, 550 k 236 / 238, 696 k 311 / 301, 1 M 451 / 407
+constexpr int kDensWide = 600000;
 template <bool KS>
 __global__ __launch_bounds__(kBlock) void k_density_wide(PV pv, GridDev g, SimParams P, NbrList L, Count nc) {
   const int n = nc.get();
