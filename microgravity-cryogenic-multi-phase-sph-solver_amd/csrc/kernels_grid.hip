@@ -53,15 +53,17 @@ __global__ __launch_bounds__(kBlock) void k_kick_drift_keys(PV pv, GridDev g, De
 }
 
 // ------------------------------------------------------------- radix sort
-// A tile's keys are ranked round by round (three barriers each), so few keys
-// take short tiles, which also spread over more CUs: a scatter of 26 k keys
-// takes 20 us with 16 rounds and 8 with 4.
+// A tile's keys are ranked round by round (three barriers each), so short tiles,
+// which also spread over more CUs, make the faster scatter; the long ones keep
+// the table of tiles small (256 counters a tile, scanned row by row and written
+// with one line per counter), which counts for more from kRsFew keys on.
+// One digit's histogram, scan and scatter, us with 4 / with 16 rounds:
+//   300 k 4.8 + 4.8 + 8.3 / 6.3 + 4.8 + 20.7, 1.2 M 7.0 + 4.9 + 11.6 / 6.9 + 4.9 + 23.9,
+//   2.2 M 9.8 + 5.5 + 18.4 / 9.2 + 4.9 + 26.7, 4.5 M 16.2 + 11.2 + 31.0 / 14.0 + 4.8 + 33.1,
+//   9.1 M 25.3 + 25.8 + 50.9 / 23.7 + 5.7 + 61.3
 constexpr int kRsThreads = 256;
 constexpr int kRsItems = 16, kRsItemsFew = 4;
-// Keys from which the long tiles are used.  A scatter of 1.2 M keys took 24 us
-// with them and 12 with short ones too, so the line can go once the sort has
-// been compared at full size with short tiles alone.
-constexpr int kRsFew = 400000;
+constexpr int kRsFew = 3000000;
 
 template <int ITEMS>
 __global__ __launch_bounds__(kRsThreads) void k_radix_hist(const uint32_t* keys, Count nc, int shift,
