@@ -173,6 +173,11 @@ __host__ __device__ inline float akinci_coh(float r, float c) {
 // RISC System/6000 processor", IBM J. Res. Dev. 34, 1990): 30 cycles for the
 // square root, 14 for a reciprocal that several quotients share, 15 a quotient.
 // y: normal, at most 2^126; x: 0 or at least kFastLow in magnitude, the quotient normal.
+// A quotient is correctly rounded if r is.  One Newton step alone does not give
+// that (the significand of all ones is the known exception, a few more depend on
+// the last bit it starts from); from v_rcp_f32's values it does, for every y:
+// tests/cpp/fast_math.hip runs all of them against the IEEE operations, all x of
+// the square root, and the quotients over every significand of y.
 struct Recip {
   float y, r;  // r: 1 / y correctly rounded
 };

@@ -6,6 +6,9 @@ outside the fast arithmetic's range (coincident and nearly coincident
 particles, an infinite temperature, fluid at rest), whose targets are done
 again with IEEE operations; tiny and large lengths that switch it off; particle
 counts on either side of the sizes where a pass takes another form."""
+import subprocess
+from pathlib import Path
+
 import numpy as np
 import pytest
 
@@ -14,6 +17,17 @@ import cabi
 pytestmark = pytest.mark.gpu
 
 FIELDS = ("x", "v", "rho", "T", "p", "a", "ab", "fw", "mw", "drho", "dTdt", "kappa")
+
+
+def test_fast_arithmetic_rounds_as_ieee():
+    """Reciprocal, division and square root of the pair loops over the range they
+    are used in: all significands, no result differs from the IEEE operation's."""
+    exe = Path(__file__).resolve().parent / "cpp" / "fast_math"
+    assert exe.exists(), "tests/cpp/fast_math is built by __graft_entry__.build()"
+    print("fast arithmetic", flush=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=100)
+    print(r.stdout, flush=True)
+    assert r.returncode == 0 and r.stdout.split() == ["0", "0", "0"], r.stdout + r.stderr
 
 
 def tank(scale=1.0, model="csf", seed=0):
