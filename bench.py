@@ -175,9 +175,9 @@ def ensemble_measure(cabi, tanks, steps, tune_steps=3):
     """The same tanks advanced `steps` steps by the per-tank loop of Solvers (the
     default launch shape), then autotuned (cryo_solver_autotune: each member
     keeps the fastest launch variant of its neighbour passes, then, where its
-    forces pass runs over LDS cell tiles, cryo_solver_autotune_tiles the fastest
-    cell-tile shape; the results are the same bits either way), then by the
-    loop again and by cryo_ensemble_run_steps
+    interface pass runs over LDS cell tiles (SPS and Akinci members; none here),
+    cryo_solver_autotune_tiles the fastest cell-tile shape; the results are the
+    same bits either way), then by the loop again and by cryo_ensemble_run_steps
     (bitwise the loop's results; the GPU test checks that), wall-clock per
     ensemble step each way; and the ensemble once more with every member in
     the precision form, the form whose slosh force meets the FP64 bar."""
@@ -193,13 +193,13 @@ def ensemble_measure(cabi, tanks, steps, tune_steps=3):
     for s in solvers:
         s.run_steps(steps)
     loop = time.perf_counter() - t0
-    def tune_member(s):
+    def tune_member(s, cfg):
         v = s.autotune(tune_steps)[0]
-        shape = s.autotune_tiles(tune_steps)[0] if (v & 1) == 0 else s.tile_shape()
-        return v, shape
+        tiles = (cfg.surface_tension == 2 or cfg.sps_turbulence) and (v & 2) == 0
+        return v, s.autotune_tiles(tune_steps)[0] if tiles else s.tile_shape()
 
     t0 = time.perf_counter()
-    tuned = [tune_member(s) for s in solvers]
+    tuned = [tune_member(s, t["cfg"]) for s, t in zip(solvers, tanks)]
     picks = [v for v, _ in tuned]
     tune = time.perf_counter() - t0
     t0 = time.perf_counter()
@@ -245,9 +245,9 @@ def ensemble_measure(cabi, tanks, steps, tune_steps=3):
         s.set_particles(t["ps"], t["lo"], t["hi"])
         s.set_frame_motion(acc=(t["a_lat"], 0.0, 0.0))
         prec.append(s)
-    for s in prec:
+    for s, t in zip(prec, tanks):
         s.run_steps(1)
-        tune_member(s)
+        tune_member(s, t["cfg"])
     t0 = time.perf_counter()
     cabi.hip_ensemble_run_steps(prec, steps)
     ens_prec = time.perf_counter() - t0

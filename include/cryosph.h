@@ -193,7 +193,9 @@ int cryo_ensemble_run_steps(cryo_solver* const* solvers, int32_t count, int64_t 
  * cryo_solver_autotune times `trial_steps` steps of each variant from the
  * solver's current state (after one untimed step each), keeps the fastest,
  * returns it in *variant (may be NULL) and each variant's milliseconds per step
- * in ms_per_step[0..3] (may be NULL), and puts the solver's state back as it was. */
+ * in ms_per_step[0..3] (may be NULL), and puts the solver's state back as it was.
+ * Where the interface pass has one form, bit 1 is left as it is and the two
+ * variants that differ in nothing else share one time. */
 int cryo_solver_set_launch_variant(cryo_solver* s, int32_t variant);
 /* Extension (no counterpart in the reference): on != 0 makes cryo_solver_run_steps
  * and cryo_ensemble_run_steps capture this solver's step as a HIP graph (one per
@@ -239,7 +241,10 @@ int cryo_solver_autotune(cryo_solver* s, int32_t trial_steps, int32_t* variant, 
  * variant, from the solver's current state (after one untimed step each),
  * keeps the fastest, returns its index in *pick (may be NULL) and each shape's
  * milliseconds per step in ms_per_step[k] (may be NULL; count entries, six
- * for the built-in list), and puts the solver's state back as it was. */
+ * for the built-in list), and puts the solver's state back as it was.  Where no
+ * launch depends on the shape (neither SPS nor Akinci, or launch variant bit 1
+ * set), one time stands for all shapes and the current one is kept if it is
+ * among them (else the first). */
 int cryo_solver_set_tile_shape(cryo_solver* s, int32_t cells_x, int32_t cells_y, int32_t cells_z);
 int cryo_solver_tile_shape(cryo_solver* s, int32_t* cells_xyz);
 int cryo_solver_autotune_tiles(cryo_solver* s, int32_t trial_steps, const int32_t* shapes, int32_t count,

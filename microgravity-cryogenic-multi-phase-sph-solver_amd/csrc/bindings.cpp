@@ -723,8 +723,9 @@ PYBIND11_MODULE(CryoSPH, m) {
         return py::make_tuple(v, py::make_tuple(ms[0], ms[1], ms[2], ms[3]));
       }, py::arg("trial_steps") = 5,
          "Times trial_steps steps of each launch variant of the neighbour passes (lanes per particle of "
-         "the forces pass; LDS cell tiles or list gathers for the interface pass), keeps the fastest, restores the state; returns (variant, "
-         "ms per step of variants 0..3).  Results do not depend on the variant.")
+         "the forces pass; LDS cell tiles or list gathers for the interface pass of SPS and Akinci runs), "
+         "keeps the fastest, restores the state; returns (variant, ms per step of variants 0..3).  Results "
+         "do not depend on the variant.")
       .def_property("launch_variant", [](Solver& S) {
         int32_t v = 0;
         check(cryo_solver_launch_variant(S.s, &v));

@@ -59,6 +59,9 @@ void launch_density(const PV& pv, const GridDev& g, const SimParams& P, const Nb
 void launch_normalize_masses(const PV& pv, const GridDev& g, const SimParams& P, int n, hipStream_t s);
 void launch_wall_bc(const PV& pv, const GridDev& g, const SimParams& P, const NbrList& L, const DevState* st, Count n,
                     hipStream_t s);
+// Whether the interface pass has the LDS-staged form (SPS and Akinci runs): without,
+// neither the tile shape nor `tiled` changes a launch.
+inline bool interface_has_tiles(const SimParams& P) { return P.st_model == 2 || P.sps; }
 int launch_interface(const PV& pv, const GridDev& g, const SimParams& P, const NbrList& L, DevState* st, Count n,
                      bool csf_mode, double* heat_partials, bool tiled, hipStream_t s);
 void launch_smooth_normals(const PV& pv, const GridDev& g, const SimParams& P, const NbrList& L, Count n,

@@ -1141,7 +1141,7 @@ int launch_interface(const PV& pv, const GridDev& g, const SimParams& P, const N
                      bool csf_mode, double* heat_partials, bool tiled, hipStream_t s) {
   const int nb = blocks_for(n.ub > 0 ? n.ub : 1);
   const int cm = csf_mode ? 1 : 0;
-  if (P.st_model != 2 && !P.sps && L.valid && g.flags) {
+  if (!interface_has_tiles(P) && L.valid && g.flags) {
     if (n.ub < (P.compensated ? kInterfaceLanesKs : kInterfaceLanes)) {
       const int sb = blocks_for(16ll * std::max(n.ub, 1));
       if (P.compensated) k_interface_lanes<true, 16><<<sb, kBlock, 0, s>>>(pv, g, P, L, st, n, cm);

@@ -1652,13 +1652,25 @@ struct cryo_solver {
     restore();
     return pick;
   }
-  // Every launch variant (ms: 4 entries).
+  // Every launch variant (ms: 4 entries).  Where the interface pass has one
+  // form, bit 1 changes no launch: it stays as it is, and its variants get the
+  // times of those without it.
   int autotune(int trials, double* ms) {
-    return time_configurations(trials, 4, launch_variant(), [this](int v) { set_launch_variant(v); }, ms);
+    if (interface_has_tiles(P))
+      return time_configurations(trials, 4, launch_variant(), [this](int v) { set_launch_variant(v); }, ms);
+    const int keep = launch_variant() & 2;
+    double t[2] = {0.0, 0.0};
+    const int v = time_configurations(trials, 2, launch_variant() & 1,
+                                      [this, keep](int k) { set_launch_variant(k | keep); }, t);
+    for (int k = 0; ms && k < 4; ++k) ms[k] = t[k & 1];
+    return v | keep;
   }
   // Tile shapes shapes[3k..3k+2], k < count, at the current launch variant;
   // shapes == nullptr: the built-in candidates below (count ignored; ms then
   // needs kTileCandidates entries).  Returns the index of the chosen shape.
+  // Where no launch depends on the shape (one form of the interface pass, or its
+  // list gathers selected), one time stands for all and the current shape stays,
+  // if it is among them.
   static constexpr int kTileCandidates = 6;
   int autotune_tiles(int trials, const int32_t* shapes, int count, double* ms) {
     static constexpr int32_t builtin[kTileCandidates * 3] = {3, 3, 3, 4, 3, 2, 4, 2, 3, 2, 3, 3, 3, 3, 2, 3, 2, 3};
@@ -1668,6 +1680,21 @@ struct cryo_solver {
       if (!tile_shape_ok(shapes[3 * k], shapes[3 * k + 1], shapes[3 * k + 2]))
         throw std::invalid_argument("autotune_tiles: tile shape " + std::to_string(k) + " out of range");
     const int keep[3] = {tile_shape[0], tile_shape[1], tile_shape[2]};
+    if (!interface_has_tiles(P) || !tile_iface) {
+      int same = 0;
+      while (same < count && !std::equal(keep, keep + 3, shapes + 3 * same)) ++same;
+      if (same == count) same = 0;
+      double t = 0.0;
+      time_configurations(
+          trials, 1, 1,
+          [&](int k) {
+            if (k == 0) set_tile_shape(shapes[3 * same], shapes[3 * same + 1], shapes[3 * same + 2]);
+            else set_tile_shape(keep[0], keep[1], keep[2]);
+          },
+          &t);
+      if (ms) std::fill(ms, ms + count, t);
+      return same;
+    }
     // the current shape is put back on an error: apply(count) means "keep"
     return time_configurations(
         trials, count, count,

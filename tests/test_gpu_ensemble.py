@@ -100,9 +100,10 @@ def test_ensemble_calls_in_a_row_and_plain_steps_between():
 
 
 def test_launch_variants_give_the_same_bits_and_autotune_restores_the_state():
-    """Every launch variant of the neighbour passes (LDS cell tiles or list
-    gathers, for forces and interface) steps a tank to the same bits; the
-    autotuner's trial steps leave no trace in the solver it tunes."""
+    """Every launch variant of the neighbour passes (lanes per particle of the
+    forces pass; LDS cell tiles or list gathers for the interface pass, which the
+    SPS and Akinci tests run) steps a tank to the same bits; the autotuner's
+    trial steps leave no trace in the solver it tunes."""
     print("test_launch_variants_give_the_same_bits_and_autotune_restores_the_state", flush=True)
     tanks = small_tanks()[:2]
     for t in tanks:
@@ -143,6 +144,41 @@ def _akinci_tank():
     return dict(cfg=cfg, fluid=fluid, ps=ps, lo=lo, hi=hi, a_lat=0.0, desc="LN2 drop, Akinci")
 
 
+def _sps_tank():
+    """Water sloshing in a box with the SPS closure: its interface pass runs over
+    LDS cell tiles with staged velocities."""
+    fluid = cabi.hip_fluid_preset("H2O")
+    cfg = cabi.default_config(dx=0.005, surface_tension=0, thermal=0, phase_change=0, density_mode=1, sps_turbulence=1,
+                              velocity_scale=1.0)
+    ps = cabi.hip_build_tank_particles(cabi.box(0.06, 0.04, 0.05), fluid, 0.005,
+                                       cabi.default_fill(include_vapor=0, fill_fraction=0.6))
+    rng = np.random.default_rng(4)
+    fl = ps.phase != cabi.WALL
+    ps.x[fl] += rng.uniform(-0.05 * 0.005, 0.05 * 0.005, size=(int(fl.sum()), 3)).astype(np.float32)
+    ps.v[fl] = rng.normal(0, 0.05, (int(fl.sum()), 3)).astype(np.float32)
+    lo, hi = ps.x.min(0) - np.float32(0.02), ps.x.max(0) + np.float32(0.02)
+    return dict(cfg=cfg, fluid=fluid, ps=ps, lo=lo, hi=hi, a_lat=0.3, desc="water box, SPS")
+
+
+def test_autotuners_time_only_what_differs():
+    """A CSF tank's interface pass has one form: the tuners leave launch-variant
+    bit 1 and the tile shape as they are, and equal launches share one time."""
+    print("test_autotuners_time_only_what_differs", flush=True)
+    s = make([small_tanks()[0]])[0]
+    s.set_launch_variant(2)
+    s.set_tile_shape(2, 3, 3)
+    v, ms = s.autotune(1)
+    assert v in (2, 3) and s.launch_variant() == v
+    assert ms[0] == ms[2] and ms[1] == ms[3] and ms[v] == min(ms) > 0
+    shape, ms = s.autotune_tiles(1)
+    assert shape == s.tile_shape() == (2, 3, 3) and len(set(ms)) == 1 and ms[0] > 0
+    shape, ms = s.autotune_tiles(1, shapes=[(1, 1, 1), (4, 2, 3)])
+    assert shape == s.tile_shape() == (1, 1, 1) and len(set(ms)) == 1
+    a = make([_akinci_tank()])[0]  # list gathers selected: no launch depends on the shape
+    a.set_launch_variant(2)
+    assert len(set(a.autotune_tiles(1)[1])) == 1 and a.tile_shape() == (3, 3, 3)
+
+
 def test_tile_shapes_give_the_same_bits_and_autotune_tiles_restores_the_state():
     """Every accepted cell-tile shape of the LDS-staged passes, from single
     cells to long thin tiles whose staged rows overflow LDS (their
@@ -150,7 +186,7 @@ def test_tile_shapes_give_the_same_bits_and_autotune_tiles_restores_the_state():
     trial steps leave no trace; shapes outside the row tables are refused."""
     print("test_tile_shapes_give_the_same_bits_and_autotune_tiles_restores_the_state", flush=True)
     shapes = HipSolver.TILE_CANDIDATES + [(1, 1, 1), (8, 1, 2), (16, 1, 1), (1, 3, 3), (2, 1, 6)]
-    for t in [small_tanks()[0], _akinci_tank()]:
+    for t in [small_tanks()[0], _akinci_tank(), _sps_tank()]:
         print(t["desc"], flush=True)
         ref = make([t])[0]
         assert ref.tile_shape() == (3, 3, 3)
