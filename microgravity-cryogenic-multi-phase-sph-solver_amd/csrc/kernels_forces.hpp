@@ -128,11 +128,13 @@ struct ForcesTarget {
   // The terms of pair (i, j); none for j == i (also used for a lane without a
   // neighbour).  FAST: correctly rounded division and square root without the
   // range handling of the IEEE sequences (the same bits within the range that
-  // unsafe() checks).  DIRECT: the terms go straight to the sums, else to o.
+  // unsafe() checks).  DIRECT: the terms go straight to the sums (the cell sweep,
+  // never FAST), else to o.
   // tvf_any / csf_any: some lane of the wave needs those terms.
   template <bool FAST, bool DIRECT>
   __device__ inline void pair(const PV& pv, const SimParams& P, int j, const PairData d, bool tvf_any, bool csf_any,
                               PairTerms<KS>& o) {
+    static_assert(!(FAST && DIRECT), "the cell sweep uses IEEE operations");
     const float h = P.kernel.h;
     const float eta2 = 0.01f * h * h;
     const V3 xj = ld3(d.x);
@@ -576,14 +578,14 @@ __global__ __launch_bounds__(kBlock, KS || ST == 2 ? 2 : (OPT || (ST == 1 && CON
         d = load(j);
         jn = entry(e + sub + 2 * G);
         PairTerms<KS> o;
-        T.template pair<decltype(fast)::value, G == 1>(pv, P, jc, c, tvf_any, csf_any, o);
-        if constexpr (G > 1) T.template add<G>(P, o, tvf_any, csf_any);
+        T.template pair<decltype(fast)::value, false>(pv, P, jc, c, tvf_any, csf_any, o);
+        T.template add<G>(P, o, tvf_any, csf_any);
       }
     };
     if (P.fast) sweep(std::true_type{});
     // (uniform over a group: its lanes hold the same sums; what each lane's own pairs met differs)
     bool again = !P.fast || T.unsafe(P);
-    if constexpr (G > 1) again = (__ballot(again) >> (lane & ~(G - 1)) & ((1ull << G) - 1)) != 0;
+    again = (__ballot(again) >> (lane & ~(G - 1)) & ((1ull << G) - 1)) != 0;
     if (again) {
       T.reset();
       sweep(std::false_type{});

@@ -1,4 +1,4 @@
-// Neighbour-loop physics on gfx950 (one thread per target particle).
+// Neighbour-loop physics on gfx950.
 //
 // The reference runs one kernel per operator (evaluate_rates,
 // sph_solver.cu:449-480).  Here operators whose inputs are ready at the same
@@ -413,7 +413,6 @@ __device__ inline IfaceNbr load_iface_nbr(const PV& pv, const SimParams& P, int 
     d.r = make_float4(nw.x, nw.y, nw.z, P.wall_colour ? pv.t.alpha[j] : 0.0f);
     if (SPS && P.no_slip) d.v = pv.t.vw[j];
   } else {
-    const float4 rec = pv.t.nrec[j];
     d.r = make_float4(pv.t.vol[j], 0.0f, 0.0f, 0.0f);  // m / rho (density pass)
     if (SPS) d.v = pv.s.v[j];
   }
@@ -725,7 +724,7 @@ __global__ __launch_bounds__(kBlock) void k_smooth_normals(PV pv, GridDev g, Sim
 // walks its particle's neighbour list reading LDS.  List entries ascend, so a
 // forward-moving row cursor maps index j to its LDS slot.  A tile whose rows
 // hold more than kTileCap particles gathers from global memory instead;
-// overflowed lists (count < 0) are left to the sweep instance of k_forces.
+// overflowed lists (count < 0) are left to the overflow instance of k_interface.
 // The tile shape (g.tx x g.ty x g.tz cells, 3 x 3 x 3 by default) is a launch
 // parameter: any shape with (ty + 2)(tz + 2) <= kTileRows staged rows and
 // ty tz <= kTileTargetRows target rows (tile_shape_ok) gives the same results.
@@ -874,8 +873,7 @@ __device__ inline int tile_round_fluid(const PV& pv, const NbrList& L, const Til
 
 
 // ---------------------------------------------- interface, LDS-staged tiles
-// Same tiles and row tables as k_forces_tiled.  Staged per particle: x with
-// phase and flags bits, and {m/rho} (fluid) or {nrm, alpha} (wall): 32 B, so
+// Staged per particle: x with phase and flags bits, and {m/rho} (fluid) or {nrm, alpha} (wall): 32 B, so
 // two workgroups fit a CU (48 B and one workgroup with SPS).  Wall normals
 // and colours are staged for walls only: the pass writes the fluid ones.
 // Writes heat_w, not its sum (k_heat_partials sums it).

@@ -35,11 +35,10 @@ __device__ inline float powf_cr(float x, float y) { return static_cast<float>(po
 // operand).  The sums therefore see the reference's order, whatever G is.
 template <int G>
 struct Lanes {
-  static_assert(G == 1 || G == 2 || G == 4 || G == 16, "a quad's parts, or a row of 16 lanes");
+  static_assert(G == 2 || G == 4 || G == 16, "a quad's parts, or a row of 16 lanes");
   // every lane of the group gets lane k's v
   template <int K>
   __device__ static inline float from(float v) {
-    if constexpr (G == 1) return v;
     constexpr int b = G == 2 ? 2 + K : K;
     constexpr int ctrl = G == 16 ? 0x150 + K : K | (K << 2) | (b << 4) | (b << 6);  // row_newbcast or quad_perm
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, 0xf, 0xf, true));
