@@ -1173,15 +1173,16 @@ void launch_heat_norm(DevState* st, const double* partials, int nb, bool active,
 
 // Lanes per particle of the forces pass: four while the chip is not full
 // (shorter chains), two beyond (each lane of a group repeats the ordered
-// additions, four times as dear in the precision form).  us with four / two:
-//   CSF  45 k 56 / 72, 60 k 65 / 76, 80 k 85 / 81, 110 k 101 / 100, 188 k 149 / 145, 600 k 403 / 356
-//   CSF, precise  26 k 67 / 88, 40 k 85 / 88, 60 k 113 / 91, 120 k 180 / 151, 600 k 682 / 513
-//   no tension  60 k 48 / 57, 120 k 72 / 77, 233 k 107 / 110, 297 k 139 / 128
-//   no tension, SPS  61 k 52 / 68, 150 k 94 / 91, 233 k 139 / 144, 297 k 183 / 160
-//   Akinci  34 k 70 / 92, 113 k 161 / 183, 217 k 265 / 270, 299 k 364 / 354, 489 k 565 / 526
+// additions, four times as dear in the precision form).  us with four / two,
+// tanks and columns in motion:
+//   CSF  45 k 56 / 73, 60 k 66 / 80, 75 k 81 / 84, 90 k 87 / 83, 188 k 149 / 145, 600 k 403 / 356
+//   CSF, precise  26 k 68 / 88, 50 k 87 / 91, 60 k 115 / 100, 120 k 180 / 151, 600 k 682 / 513
+//   no tension  76 k 45 / 59, 123 k 73 / 70, 150 k 74 / 78, 233 k 103 / 106, 297 k 130 / 124
+//   no tension, SPS  76 k 55 / 71, 90 k 73 / 73, 123 k 88 / 83, 151 k 102 / 91, 233 k 139 / 143, 297 k 176 / 158
+//   Akinci  90 k 133 / 156, 136 k 183 / 190, 256 k 302 / 312, 345 k 391 / 379
 // `other` takes the other count.
 int forces_lanes(const SimParams& P, bool csf_mode, int n, bool other) {
-  const int below = P.compensated ? 50000 : csf_mode ? 75000 : 250000;
+  const int below = P.compensated ? 50000 : csf_mode || P.sps ? 80000 : 250000;
   return (n < below) != other ? 4 : 2;
 }
 

@@ -161,7 +161,7 @@ def beside(ps, dx, n):
                             cat(ps.flags, z), None)
 
 
-@pytest.mark.parametrize("n", [21_000, 30_000, 65_000, 80_000, 160_000, 310_000, 610_000, 2_999_999, 3_000_000])
+@pytest.mark.parametrize("n", [21_000, 30_000, 65_000, 81_000, 160_000, 310_000, 610_000, 2_999_999, 3_000_000])
 @pytest.mark.parametrize("compensated", [0, 1])
 @pytest.mark.parametrize("crowd", [False, True])
 def test_the_form_a_size_selects_changes_no_bit(crowd, compensated, n):
