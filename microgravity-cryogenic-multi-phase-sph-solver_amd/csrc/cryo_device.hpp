@@ -722,21 +722,16 @@ __host__ __device__ inline void df_add(float& x, float& lo, float d) {
 // wall pass.
 struct alignas(64) PairRec {
   float4 x;  // position, phase (int bits)
-  float4 q;  // {p, m, rho, T} fluid; {p, p_wv, rho_tvf, T} wall (as nrec)
+  float4 q;  // {p, m, rho, T} fluid; {p, p_wv, rho_tvf, T} wall (rho_tvf: the density liquid targets' transport velocity takes)
   float4 v;  // velocity, V = m / rho (fluid); no-slip ghost velocity, 0 (wall)
   float4 t;  // transport velocity, transport volume 1 / sigma (fluid, transport velocity on)
 };
 struct Scratch {
   float4 *a, *ab, *ns, *vw, *fw, *mw;
   float *p, *drho, *dTdt, *sigma, *kappa, *nu_t, *alpha, *wall_w, *heat_w, *out_m, *out_h, *w_norm, *p_wv, *rmin;
-  // Neighbour record of one rates evaluation, so a pair loop gathers one
-  // float4 instead of four scalars: {p, m, rho, T} for fluid particles
-  // (written by the density pass), {p, p_wv, rho_tvf, T} for walls (wall
-  // pass; rho_tvf is the wall density liquid targets use for the transport
-  // velocity).
-  float4* nrec;
-  // V = m / rho of each fluid particle for one rates evaluation (density
-  // pass): the pair loops read it instead of dividing per pair.
+  // Of one rates evaluation: V = m / rho of each fluid particle (density pass),
+  // which the pair loops read instead of dividing per pair; of a wall, rec.q.z
+  // (wall pass).
   float* vol;
   PairRec* rec;
 };

@@ -173,7 +173,7 @@ __device__ inline float tvf_K(const PV& pv, const SimParams& P, int i) {
 // The wall density a transport owner of phase ph uses for wall j.
 __device__ inline float tvf_rho_w(const PV& pv, const SimParams& P, uint8_t ph, float Ti, int j) {
   if (ph == kVapor) return (pv.t.p_wv[j] - (P.p_bg - P.vapor_K)) / (P.gas_R * Ti);
-  return pv.t.nrec[j].z;  // rho0 max(ratio, 0.5)^(1/gamma), evaluated by the wall pass
+  return pv.t.vol[j];  // rho0 max(ratio, 0.5)^(1/gamma), evaluated by the wall pass
 }
 __global__ __launch_bounds__(kBlock) void k_adj_prep(PV pv, SimParams P, AdjArgs A, const DevState* st, int n) {
   const int i = gtid();

@@ -82,7 +82,6 @@ __device__ inline void density_finish(const PV& pv, const SimParams& P, int i, c
   pv.t.p[i] = p;
   const float4 q = make_float4(p, mi, rho, Ti);
   const float V = mi / rho;
-  pv.t.nrec[i] = q;
   pv.t.vol[i] = V;
   const float4 v = pv.s.v[i], vt = pv.s.vt[i];
   pv.t.rec[i] = PairRec{make_float4(xi.x, xi.y, xi.z, __int_as_float(ph)), q, make_float4(v.x, v.y, v.z, V),
@@ -383,7 +382,7 @@ __global__ __launch_bounds__(kBlock) void k_wall_bc(PV pv, GridDev g, SimParams 
     rho_tvf = P.rho0[0] * powf_cr(ratio > 0.5f ? ratio : 0.5f, 1.0f / P.tait_gamma);
   }
   const float4 q = make_float4(pw[0], pw[1], rho_tvf, pv.s.T[i]);
-  pv.t.nrec[i] = q;
+  pv.t.vol[i] = rho_tvf;
   float4 ghost = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   if (P.no_slip && swt > 0.0f) ghost = st3(V3(sv) * (-1.0f / swt));
   pv.t.rec[i] = PairRec{make_float4(xi.x, xi.y, xi.z, __int_as_float(kWall)), q, ghost, st3(V3{0, 0, 0})};
@@ -899,8 +898,8 @@ __global__ __launch_bounds__(kTileThreads) void k_interface_tiled(PV pv, GridDev
   if (nfl0 == 0 && ntarget <= kTileThreads) return;  // uniform over the block
   if (staged) {
     // Named slots, not arrays (arrays of them are not kept in registers).
-    // First pass: position, phase, flags; second: the record the phase
-    // selects (a wall's normal and colour, a fluid particle's m and rho).
+    // First pass: position, phase, flags; second: what the phase selects (a
+    // wall's normal and colour, a fluid particle's volume).
     struct Slot {
       float4 x, r, v;
       int j, bits;
@@ -921,9 +920,8 @@ __global__ __launch_bounds__(kTileThreads) void k_interface_tiled(PV pv, GridDev
       if (s < M) {
         const bool wall = (q.bits & 0xff) == kWall;
         // (fluid normals and colours are being written by this pass)
-        const float4* src = wall ? pv.s.nrm : pv.t.nrec;  // two global arrays: a pointer select is fine
-        q.r = src[q.j];
-        q.a = (wall && P.wall_colour) ? pv.t.alpha[q.j] : 0.0f;
+        if (wall) q.r = pv.s.nrm[q.j];
+        if (!wall || P.wall_colour) q.a = (wall ? pv.t.alpha : pv.t.vol)[q.j];  // two global arrays: a pointer select is fine
         q.v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         if (SPS && (!wall || P.no_slip)) q.v = (wall ? pv.t.vw : pv.s.v)[q.j];
       }
@@ -934,7 +932,7 @@ __global__ __launch_bounds__(kTileThreads) void k_interface_tiled(PV pv, GridDev
       if (s < M) {
         const bool wall = (q.bits & 0xff) == kWall;
         s_x[s] = make_float4(q.x.x, q.x.y, q.x.z, __int_as_float(q.bits));
-        s_r[s] = wall ? make_float4(q.r.x, q.r.y, q.r.z, q.a) : make_float4(q.r.y / q.r.z, 0.0f, 0.0f, 0.0f);
+        s_r[s] = wall ? make_float4(q.r.x, q.r.y, q.r.z, q.a) : make_float4(q.a, 0.0f, 0.0f, 0.0f);
         if (SPS) s_v[s] = q.v;
       }
     };

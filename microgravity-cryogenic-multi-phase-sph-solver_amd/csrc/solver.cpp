@@ -225,7 +225,7 @@ struct cryo_solver {
   DevBuf<uint8_t> phase_[2], flags_[2];
   DevBuf<uint32_t> id_[2];
   int set = 0;
-  DevBuf<float4> a, ab, ns, vw, fw, mw, nrec;
+  DevBuf<float4> a, ab, ns, vw, fw, mw;
   DevBuf<float> p, drho, dTdt, sigma, kappa, nu_t, alpha, wall_w, heat_w, out_m, out_h, w_norm, p_wv, rmin, vol;
   DevBuf<PairRec> rec;  // neighbour records of the current rates evaluation
   // grid and scans
@@ -412,7 +412,7 @@ struct cryo_solver {
                    rho_[k].get(), T_[k].get(), phase_[k].get(), flags_[k].get(), id_[k].get(), xlo_[k].get()};
     pv.t = Scratch{a.get(), ab.get(), ns.get(), vw.get(), fw.get(), mw.get(), p.get(), drho.get(), dTdt.get(),
                    sigma.get(), kappa.get(), nu_t.get(), alpha.get(), wall_w.get(), heat_w.get(), out_m.get(),
-                   out_h.get(), w_norm.get(), p_wv.get(), rmin.get(), nrec.get(), vol.get(), rec.get()};
+                   out_h.get(), w_norm.get(), p_wv.get(), rmin.get(), vol.get(), rec.get()};
     pv.capacity = capacity;
     return pv;
   }
@@ -449,8 +449,7 @@ struct cryo_solver {
       f(id_[k], k == set);
       if (cfg.compensated_sums) f(xlo_[k], k == set);
     }
-    f(a, true); f(ab, true); f(ns, true); f(vw, true); f(fw, true); f(mw, true); f(nrec, false); f(vol, false);
-    f(rec, false);
+    f(a, true); f(ab, true); f(ns, true); f(vw, true); f(fw, true); f(mw, true); f(vol, false); f(rec, false);
     f(p, true); f(drho, true); f(dTdt, true); f(sigma, true); f(kappa, true); f(nu_t, true); f(alpha, true);
     f(wall_w, true); f(heat_w, true); f(out_m, true); f(out_h, true); f(w_norm, true); f(p_wv, true); f(rmin, true);
   }
@@ -1157,7 +1156,7 @@ struct cryo_solver {
   // optionally `a` (at step boundaries) and the step's sort permutation (taped
   // post-sort states).
   struct Snap {
-    DevBuf<float4> x, v, vt, nrm, a, ab, nrec, xlo;
+    DevBuf<float4> x, v, vt, nrm, a, ab, xlo;
     DevBuf<float> m, m0, rho, T, vol;
     DevBuf<int> lidx, lcnt, coff;  // neighbour lists and cell table of a taped rates evaluation
     DevBuf<uint8_t> cflags;
@@ -1199,7 +1198,7 @@ struct cryo_solver {
       CopyBatch cb(*this);
       d2d(z.rho.get(), q.rho, n), d2d(z.nrm.get(), q.nrm, n);
       snap_save_scratch(z);
-      fit(z.nrec, n), d2d(z.nrec.get(), t.nrec, n), fit(z.vol, n), d2d(z.vol.get(), t.vol, n);
+      fit(z.vol, n), d2d(z.vol.get(), t.vol, n);
       fit(z.lidx, nl), d2d(z.lidx.get(), nbr_idx.get(), static_cast<int>(nl));
       fit(z.lcnt, n), d2d(z.lcnt.get(), nbr_count.get(), n);
       fit(z.coff, g.num_cells + 2), d2d(z.coff.get(), cell_off.get(), g.num_cells + 2);
@@ -1214,7 +1213,7 @@ struct cryo_solver {
       CopyBatch cb(*this);
       snap_load(z, false);
       snap_load_scratch(z);
-      d2d(t.nrec, z.nrec.get(), z.n), d2d(t.vol, z.vol.get(), z.n);
+      d2d(t.vol, z.vol.get(), z.n);
       d2d(nbr_idx.get(), z.lidx.get(), static_cast<int>(nl)), d2d(nbr_count.get(), z.lcnt.get(), z.n);
       d2d(cell_off.get(), z.coff.get(), g.num_cells + 2), d2d(cell_flags.get(), z.cflags.get(), g.num_cells);
     }
