@@ -50,6 +50,7 @@ HBM_PEAK_GBS = 8000.0
 
 C2_DX = 0.007  # the workload the committed counter profiles were taken on
 VALU_CLOCK_HZ = 2.4e9  # MI355X peak engine clock
+VALU_CYCLES = 3  # a wave's add, multiply or FMA on one SIMD (measured 2.5 to 2.9)
 SIMDS = 1024  # 256 CUs x 4 SIMDs
 
 
@@ -495,17 +496,18 @@ def main():
     step_bytes = n_fluid * STEP_BYTES["fluid"] + n_wall * STEP_BYTES["wall"]
     # HBM roofline on algorithmic bytes (live kernel time), and the roof that
     # binds: the kernel's VALU issue share, VALU instructions per launch (from
-    # the committed counter profile of this workload) x 4 cycles per wave64
-    # instruction over the SIMD-cycles of the live launch time.  Counter-based
-    # fields are given only for the workload the profiles were taken on.
+    # the committed counter profile of this workload) x the cycles a plain
+    # multiply or FMA takes over the SIMD-cycles of the live launch time: a lower
+    # bound, compares, reciprocals and roots take longer.  Counter-based fields
+    # are given only for the workload the profiles were taken on.
     on_profile = abs(a.dx - C2_DX) < 1e-9
     traffic = profile_column("hbm_traffic_c2.txt", "k_forces<", 1) if on_profile else None
     valu_instr = profile_column("valu_l2_c2.txt", "k_forces<", 2) if on_profile else None
-    valu_frac = (valu_instr * 4 / SIMDS / (forces_ms * 1e-3 * VALU_CLOCK_HZ)) if valu_instr else None
+    valu_frac = (valu_instr * VALU_CYCLES / SIMDS / (forces_ms * 1e-3 * VALU_CLOCK_HZ)) if valu_instr else None
     tfrac = (traffic / (forces_ms * 1e-3) / 1e9 / HBM_PEAK_GBS) if traffic else None
     if valu_frac is None:
         limiter = None
-    elif valu_frac >= 0.8 or (tfrac or 0.0) >= 0.8:
+    elif valu_frac >= 0.7 or (tfrac or 0.0) >= 0.8:
         limiter = "VALU issue" if valu_frac >= (tfrac or 0.0) else "HBM traffic"
     else:
         limiter = "latency: neither the VALU nor the HBM roof is reached"
