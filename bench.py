@@ -518,7 +518,7 @@ def main():
                 if traffic else None,
                 "traffic_frac": tfrac,
                 "valu_frac": valu_frac,
-                "valu_source": "profiles/valu_l2_c2.txt (SQ_INSTS_VALU per launch) over the live kernel time"
+                "valu_source": "profiles/valu_l2_c2.txt (SQ_INSTS_VALU per launch, mean of 24) over the live kernel time"
                 if valu_frac is not None else None,
                 "limiter": limiter,
                 "kernel": "k_forces (transport velocity + momentum + wall loads + continuity + dt "

@@ -513,10 +513,13 @@ __device__ inline void publish_maxima(DevState* st, Maxima mx) {
 // registers alone (<= 128, four waves per SIMD) set the occupancy, and any
 // number of particles spreads evenly over the chip.  It replaced one thread
 // per particle over LDS-staged cell tiles (159 KB, 1.35 waves per SIMD, five
-// atomics a wave): 2.2 M-particle column 2308 -> 840 us per launch, 1.2 M
-// two-phase sphere 1826 -> 662, 188 k tank 324 -> 147, 26 k tank 206 -> 48,
-// precision form at 293 k 724 -> 287.  Bound by the gathers (a tag look-up per
-// lane and 16 bytes) and the pair arithmetic about equally.
+// atomics a wave).  us a launch by kernel traces, before and now: 2.2 M-particle
+// column in motion 2274 / 831, the benchmark's column in its first 24 launches
+// 1907 / 1015 (nearly at rest: up to a quarter of its fluid targets meet tiny
+// numerators and are swept twice), 1.2 M two-phase sphere 1828 / 661, 188 k tank
+// 323 / 142, 26 k tank 203 / 48, precision form at 293 k 713 / 281.  Bound by the
+// pair arithmetic (84 % of the VALU's issue at 3 cycles an instruction) and the
+// gathers (a tag look-up per lane and 16 bytes).
 template <int ST, bool CONT, bool THERMAL, bool KS, bool OPT, int G>
 __global__ __launch_bounds__(kBlock, KS || ST == 2 ? 2 : (OPT || (ST == 1 && CONT) ? 3 : 4)) void k_forces(PV pv, SimParams P, NbrList L, DevState* st, Count nc) {
   constexpr int kSpan = kBlock / G;
