@@ -117,7 +117,8 @@ def test_lengths_beyond_the_fast_range(scale):
     check(fluid, cfg, ps, dx, 0, steps=1)
 
 
-@pytest.mark.parametrize("n", [2047, 2049, 59_999, 60_000, 99_999, 100_000, 119_999, 249_999, 250_000, 399_999, 400_000, 599_999, 600_000, 700_000])
+@pytest.mark.parametrize("n", [2047, 2049, 59_999, 60_000, 79_999, 80_000, 99_999, 100_000, 119_999, 139_999, 140_000,
+                               249_999, 250_000, 299_999, 300_000, 399_999, 400_000, 599_999, 600_000, 700_000])
 def test_both_sides_of_the_size_rules(n):
     """A heated, superheated two-phase tank of exactly n particles: every pass of
     a step with phase change.  Without transport velocity, whose wall density
